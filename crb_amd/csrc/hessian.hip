@@ -21,7 +21,9 @@
 //  * in-place path (k_syrk16p): a loading thread reads a 4-token x
 //    8-channel unit with four 16-byte loads and transposes it in registers
 //    with v_perm_b32 before one 8-byte LDS store per channel.
-// The first two issue the same MFMAs on the same operands for the same
+// Calls with few 256 x 256 tiles run on 64 x 64 tiles instead (k_syrk16s),
+// with token-major stages whatever the alignment.
+// The first two and k_syrk16s issue the same MFMAs on the same operands for the same
 // token splits, so their sums are bitwise equal.
 #include <stdlib.h>
 
@@ -32,17 +34,6 @@
 #include "common.h"
 
 namespace crbq {
-
-constexpr int HT = 128;      // output tile of the fp32-input kernel
-constexpr int HK32 = 16;     // tokens per LDS stage (fp32 input)
-
-__device__ __forceinline__ void tile_of(int idx, int nt, int& ti, int& tj) {
-  // idx over the upper triangle row by row: row ti has nt - ti tiles
-  int i = 0, rem = idx;
-  while (rem >= nt - i) { rem -= nt - i; ++i; }
-  ti = i;
-  tj = i + rem;
-}
 
 template <typename T8>
 __device__ __forceinline__ f4_t mfma16(T8 a, T8 b, f4_t c);
@@ -850,61 +841,281 @@ static void sum_splits(const float* P, int nsplit, int64_t C, float* S, int64_t 
                                                                       nt, vec);
 }
 
-// fp32 inputs: LDS in natural token-major layout, A[i][k] = X[k][i].
-__global__ __launch_bounds__(256) void k_syrk32(const float* __restrict__ X, int64_t ntok,
-                                                int64_t ldx, int C, float* S, int64_t lds,
-                                                int nt) {
-  __shared__ float Xs[2][HK32][HT + 4];
-  int ti, tj;
-  tile_of(blockIdx.x, nt, ti, tj);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  const bool diag = ti == tj;
-  f4_t acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
-  for (int64_t t0 = 0; t0 < ntok; t0 += HK32) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int idx = tid + 256 * e;           // 0..4095 = 2 sides x 16 tokens x 128 ch
-      const int side = idx >> 11, k = (idx >> 7) & 15, c = idx & 127;
-      if (diag && side) continue;
-      const int gc = (side ? tj : ti) * HT + c;
-      const int64_t t = t0 + k;
-      Xs[side][k][c] = (t < ntok && gc < C) ? X[t * ldx + gc] : 0.f;
+// fp32 inputs (v_mfma_f32_16x16x4_f32): no LDS on the way to the matrix
+// units.  A lane of the MFMA holds one token (lane >> 4) of one channel
+// (lane & 15) per operand; here lane l takes NS = 2 or 4 consecutive
+// channels NS * (l & 15) .. of its token with one 8- or 16-byte load, its
+// element s being the operand of the s-th 16 x 16 subtile: the subtiles
+// interleave the wavefront's 16 * NS channels instead of splitting them into
+// ranges, which only permutes the output index (and makes a lane's NS
+// subtile columns consecutive, so S is updated with vector accesses).
+// A workgroup covers 16 NS x 16 NS outputs; its KS wavefronts split the
+// tokens (chunks in turn) and their sums meet in LDS in wavefront order:
+// small inputs have few output tiles, so the token range is what fills the
+// chip.  (128 x 128 tiles of one token range staged in LDS took 101-180 us
+// for 512 tokens of 768 channels, on 21 workgroups, and 1609 us for 4096 x
+// 4096; this takes 11 and 730.)  Each wavefront loads one chunk (16 tokens,
+// or 32 with 2 channels per lane) ahead in registers.  Channels at or beyond
+// C are read from channel 0: an output depends on its own two channels only,
+// and theirs are not stored.  VEC: X is aligned, C and ldx multiples of 4.
+// Bound by the operand loads from L2 (6 TB/s on 64 x 64 tiles, 0.63-0.7 of
+// the fp32 matrix rate).
+
+template <int NS, bool VEC>
+__device__ __forceinline__ void s32_load(const float* __restrict__ p, int C, int c0,
+                                         float (&v)[NS]) {
+  if constexpr (VEC) {
+    if constexpr (NS == 4) {
+      const float4 q = *(const float4*)(p + (c0 < C ? c0 : 0));
+      v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+      const float2 q = *(const float2*)(p + (c0 < C ? c0 : 0));
+      v[0] = q.x; v[1] = q.y;
     }
-    __syncthreads();
-    const int sj = diag ? 0 : 1;
+  } else {
 #pragma unroll
-    for (int kk = 0; kk < HK32; kk += 4) {
-      const int kr = kk + (lane >> 4), c16 = lane & 15;
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = Xs[0][kr][wm + i * 16 + c16];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Xs[sj][kr][wn + j * 16 + c16];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();
+    for (int e = 0; e < NS; ++e) v[e] = p[c0 + e < C ? c0 + e : 0];
   }
+}
+
+template <int NS, int KS, bool VEC>
+__global__ __launch_bounds__(64 * KS) void k_syrk32(const float* __restrict__ X, int64_t ntok,
+                                                    int64_t ldx, int C, float* S, int64_t lds,
+                                                    int nt, int vs) {
+  constexpr int TILE = 16 * NS;
+  constexpr int NK = NS == 2 ? 8 : 4, S32_CH = 4 * NK;     // k-steps and tokens per chunk
+  int ti, tj;
+  upper_tile(blockIdx.x, nt, ti, tj);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int ci = ti * TILE, cj = tj * TILE;
+  const int c16 = lane & 15, kr = lane >> 4;
+  f4_t acc[NS][NS];
+#pragma unroll
+  for (int i = 0; i < NS; ++i)
+#pragma unroll
+    for (int j = 0; j < NS; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+  float a[NK][NS], b[NK][NS];
+  auto load = [&](int64_t t0) {
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      int64_t t = t0 + 4 * k + kr;
+      t = t < ntok ? t : ntok - 1;
+      s32_load<NS, VEC>(X + t * ldx, C, ci + NS * c16, a[k]);
+      s32_load<NS, VEC>(X + t * ldx, C, cj + NS * c16, b[k]);
+    }
+  };
+  const int64_t step = (int64_t)S32_CH * KS;
+  int64_t t0 = (int64_t)S32_CH * wave;
+  if (t0 < ntok) load(t0);
+  for (; t0 < ntok; t0 += step) {
+    float ua[NK][NS], ub[NK][NS];
+    const bool whole = t0 + S32_CH <= ntok;
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+#pragma unroll
+      for (int e = 0; e < NS; ++e) {
+        const bool ok = whole || t0 + 4 * k + kr < ntok;
+        ua[k][e] = ok ? a[k][e] : 0.f;
+        ub[k][e] = ok ? b[k][e] : 0.f;
+      }
+    load(t0 + step < ntok ? t0 + step : t0);
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+#pragma unroll
+      for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ua[k][i], ub[k][j], acc[i][j], 0, 0, 0);
+  }
+  // element (row 4 (lane >> 4) + r, column lane & 15) of subtile (i, j) is
+  // output (ci + NS * row + i, cj + NS * column + j)
+  auto put = [&](int i, int r, const float (&v)[NS]) {
+    const int gi = ci + NS * (4 * kr + r) + i, gj = cj + NS * c16;
+    if (gi >= C) return;
+    float* p = S + (int64_t)gi * lds + gj;
+    if (vs && gi <= gj && gj + NS <= C) {
+      if constexpr (NS == 4) {
+        float4 q = *(float4*)p;
+        q.x += v[0]; q.y += v[1]; q.z += v[2]; q.w += v[3];
+        *(float4*)p = q;
+      } else {
+        float2 q = *(float2*)p;
+        q.x += v[0]; q.y += v[1];
+        *(float2*)p = q;
+      }
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+      if (gi <= gj + j && gj + j < C) p[j] = p[j] + v[j];
+  };
+  __shared__ float red[KS][NS * 4][NS][64];
+#pragma unroll
+  for (int i = 0; i < NS; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < NS; ++j) red[wave][i * 4 + r][j][lane] = acc[i][j][r];
+  __syncthreads();
+  // row slice q = 4 i + r by wavefront q % KS
+#pragma unroll
+  for (int q0 = 0; q0 < NS * 4; q0 += KS) {
+    const int q = q0 + wave;
+    if (q >= NS * 4) continue;
+    float v[NS];
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      float t = red[0][q][j][lane];
+#pragma unroll
+      for (int w = 1; w < KS; ++w) t += red[w][q][j][lane];
+      v[j] = t;
+    }
+    put(q >> 2, q & 3, v);
+  }
+}
+
+// 16-bit inputs with few output tiles (small channel counts and short
+// calls, e.g. one calibration sample at a time): 64 x 64 upper tiles, 4
+// wavefronts of 32 x 32 outputs, straight from the token-major X.  On the 256 x 256
+// tiles of k_syrk16k a 768-channel call runs 6 workgroups, whatever its
+// token count.  A stage is 64 tokens of the tile's two 64-channel panels
+// (16 KB), loaded into registers SM_AHEAD stages ahead (these calls are too
+// short to hide memory latency any other way), stored to one of two LDS
+// buffers as token rows of 128 bytes and read with LDS transpose reads; the
+// 32-byte groups of a row are XOR-permuted by bits 1 and 3 of the row, so
+// the 8 rows half a wavefront reads land on distinct banks.  The MFMAs and
+// their order per output are those of k_syrk16k, and the token splits are
+// chosen the same way, so the sums are bitwise equal.
+// FAST: C and ldx are multiples of 8 and X is 16-byte aligned; otherwise
+// the 8 channels of a chunk are one unaligned load, one by one past C.
+constexpr int SM_T = 64;           // tile
+constexpr int SM_AHEAD = 3;
+
+__device__ __forceinline__ int sm_swz(int t) { return (((t >> 1) & 1) | ((t >> 2) & 2)) << 5; }
+
+template <typename T8>
+__device__ __forceinline__ T8 sm_frag(const char* p) {
+  typedef __attribute__((address_space(3))) const char lchar;
+  lchar* q = (lchar*)(const void*)p;
+  const tr4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr4_t*)(q));
+  const tr4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_tr4_t*)(q + 4 * SM_T * 2));
+  struct P { tr4_t a, b; } v{lo, hi};
+  return __builtin_bit_cast(T8, v);
+}
+
+template <typename T8, bool FAST>
+__global__ __launch_bounds__(256) void k_syrk16s(const uint16_t* __restrict__ X, int64_t ldx,
+                                                 int64_t ntok, int64_t tpad, int C, float* S,
+                                                 int64_t lds, int nt, int64_t span, float* P) {
+  __shared__ __attribute__((aligned(128))) uint16_t Xs[2][2][KQ][SM_T];   // [buffer][panel]
+  int ti, tj;
+  upper_tile(blockIdx.x, nt, ti, tj);
+  const int64_t k_beg = (int64_t)blockIdx.y * span;
+  const int64_t k_end = k_beg + span < tpad ? k_beg + span : tpad;
+  const int nch = k_end > k_beg ? (int)((k_end - k_beg) / KQ) : 0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // loader: chunk e of a stage (panel e >> 1): row 32 (e & 1) + tid / 8,
+  // channels 8 (tid & 7) ..
+  const int lrow = tid >> 3, lch = (tid & 7) * 8;
+  uint4 buf[SM_AHEAD][4];
+  auto load = [&](int st, uint4 (&u)[4]) {
+    const int64_t t0 = k_beg + (int64_t)(st < nch ? st : nch - 1) * KQ;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t t = t0 + 32 * (e & 1) + lrow;
+      const uint16_t* p = X + (t < ntok ? t : ntok - 1) * ldx;
+      const int c = ((e >> 1) ? tj : ti) * SM_T + lch;
+      if constexpr (FAST) {
+        u[e] = *(const uint4*)(p + (c < C ? c : 0));
+      } else {
+        if (c + 8 <= C) {
+          __builtin_memcpy(&u[e], p + c, 16);      // a load of 2-byte alignment
+        } else {
+          uint32_t h[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) h[k] = p[c + k < C ? c + k : 0];
+          u[e] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16),
+                            h[6] | (h[7] << 16));
+        }
+      }
+    }
+  };
+  auto store = [&](int st, const uint4 (&u)[4]) {
+    const int64_t t0 = k_beg + (int64_t)st * KQ;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 32 * (e & 1) + lrow;
+      const bool ok = t0 + row < ntok;          // rows past the end are zeros
+      uint4 v;
+      v.x = ok ? u[e].x : 0u; v.y = ok ? u[e].y : 0u;
+      v.z = ok ? u[e].z : 0u; v.w = ok ? u[e].w : 0u;
+      *(uint4*)((char*)&Xs[st & 1][e >> 1][row][0] + ((lch * 2) ^ sm_swz(row))) = v;
+    }
+  };
+  // fragments: lane (group gq, s) addresses row 8 gq + s / 4 at channel
+  // RB + 4 (s % 4) of its 32-token slice
+  const int gq = lane >> 4, sl = lane & 15;
+  const int trow = 8 * gq + (sl >> 2), fsw = sm_swz(trow);
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  int aoff[2], boff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    aoff[i] = trow * SM_T * 2 + (((wm + 16 * i + 4 * (sl & 3)) * 2) ^ fsw);
+    boff[i] = (KQ + trow) * SM_T * 2 + (((wn + 16 * i + 4 * (sl & 3)) * 2) ^ fsw);
+  }
+  f4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+  if (nch > 0) {
+#pragma unroll
+    for (int d = 0; d < SM_AHEAD; ++d) load(d, buf[d]);
+  }
+  for (int c0 = 0; c0 < nch; c0 += SM_AHEAD) {
+#pragma unroll
+    for (int d = 0; d < SM_AHEAD; ++d) {
+      const int c = c0 + d;
+      if (c >= nch) break;
+      store(c, buf[d]);
+      load(c + SM_AHEAD, buf[d]);
+      // one barrier per stage: buffer c & 1 was last read in stage c - 2,
+      // which every wavefront left before the barrier of stage c - 1
+      sync_lds();
+      const char* cur = (const char*)&Xs[c & 1][0][0][0];
+#pragma unroll
+      for (int h = 0; h < KQ / 32; ++h) {
+        const char* q = cur + h * 32 * SM_T * 2;
+        T8 fa[2], fb[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          fa[i] = sm_frag<T8>(q + aoff[i]);
+          fb[i] = sm_frag<T8>(q + boff[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma16<T8>(fa[i], fb[j], acc[i][j]);
+      }
+    }
+  }
+  // as syrk_store: split 0 adds into S, split s > 0 writes P[s - 1]
+  const bool part = P && blockIdx.y > 0;
+  float* out = part ? P + (size_t)(blockIdx.y - 1) * (size_t)C * lds : S;
   const int c16 = lane & 15, r4 = (lane >> 4) * 4;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int gi = ti * HT + wm + i * 16 + r4 + r;
-        const int gj = tj * HT + wn + j * 16 + c16;
+        const int gi = ti * SM_T + wm + i * 16 + r4 + r;
+        const int gj = tj * SM_T + wn + j * 16 + c16;
         if (gi < C && gj < C && gi <= gj) {
-          float* p = S + (int64_t)gi * lds + gj;
-          *p = *p + acc[i][j][r];
+          float* q = out + (int64_t)gi * lds + gj;
+          *q = part ? acc[i][j][r] : *q + acc[i][j][r];
         }
       }
 }
@@ -1161,6 +1372,82 @@ static int syrk_xt(const uint16_t* X, int64_t ld, int64_t ntok, bool tmaj, int64
 }
 }  // namespace crbq
 
+namespace crbq {
+// fp32 inputs.  32 x 32 tiles (2 channels per lane, 8 wavefronts splitting
+// the tokens) up to 2048 channels, 64 x 64 tiles (4 channels, 4 wavefronts)
+// above, where there are enough of them to fill the chip and the operand
+// traffic per product counts: measured (us, 32 against 64) 10.9 / 15.8 at
+// 768 channels x 512 tokens, 50.5 / 77 at 1530 x 1024, 130 / 146 at 2048 x
+// 2048, 56 / 50 at 2560 x 512, 829 / 732 at 4096 x 4096.
+static int syrk32(const float* X, int64_t ntok, int64_t ldx, int64_t C, float* S, int64_t lds,
+                  hipStream_t s) {
+  const bool vec = (C & 3) == 0 && (ldx & 3) == 0 && (((uintptr_t)X) & 15) == 0;
+  const int vs = (lds & 3) == 0 && (((uintptr_t)S) & 15) == 0;
+  const bool narrow = C <= 2048;
+  const int64_t nt = (C + (narrow ? 31 : 63)) / (narrow ? 32 : 64);
+  if (nt * (nt + 1) / 2 > 0x7fffffff) return CRBQ_ERR_ARG;
+  const unsigned grid = (unsigned)(nt * (nt + 1) / 2);
+#define CRBQ_S32_GO(NS_, KS_, V_) \
+  k_syrk32<NS_, KS_, V_><<<grid, 64 * KS_, 0, s>>>(X, ntok, ldx, (int)C, S, lds, (int)nt, vs)
+  if (narrow) {
+    if (vec) CRBQ_S32_GO(2, 8, true); else CRBQ_S32_GO(2, 8, false);
+  } else {
+    if (vec) CRBQ_S32_GO(4, 4, true); else CRBQ_S32_GO(4, 4, false);
+  }
+#undef CRBQ_S32_GO
+  CRBQ_LAUNCH_CHECK();
+  return CRBQ_OK;
+}
+
+// Whether a 16-bit call runs on 64 x 64 tiles: modelled microseconds of
+// both kernels.  k_syrk16s: 8 for the launch and S, then the larger of its
+// stages' latency (0.3 each) and its operand stream (128 channels per tile
+// and token at 10 TB/s); k_syrk16k: 26 for the launch and a 256 x 256 tile of
+// S, and 1.75 per stage and round.  Measured (us, k_syrk16s / k_syrk16k): 9.2
+// / 31.6 at 768 channels x 512 tokens, 41 / 86 at 768 x 16384, 587 / 450 at
+// 768 x 262144, 33 / 76 at 2048 x 2048, 96 / 89 at 2048 x 8192, 57 / 80 at
+// 3072 x 2048, 34 / 53 at 4096 x 512, 92 / 81 at 4096 x 2048.
+static bool syrk16_small(int64_t ntok, int64_t C) {
+  const int cus = num_cus();
+  const int64_t tpad = (ntok + KQ - 1) / KQ * KQ;
+  const int64_t ns = choose_splits(tpad, C, cus);
+  const double stages = (double)((tpad / KQ + ns - 1) / ns);
+  const int64_t n64 = (C + SM_T - 1) / SM_T, n256 = (C + ST - 1) / ST;
+  const double stream = (double)(n64 * (n64 + 1) / 2) * (double)tpad * (4.0 * SM_T) / 10e6;
+  const double ts = 8.0 + (stream > 0.3 * stages ? stream : 0.3 * stages);
+  const int64_t rounds = (n256 * (n256 + 1) / 2 * ns + cus - 1) / cus;
+  return ts <= 26.0 + 1.75 * stages * (double)rounds;
+}
+static int syrk16s(const uint16_t* X, int64_t ldx, int64_t ntok, bool fast, int64_t C, float* S,
+                   int64_t lds, float* Pbuf, size_t pcap, int dtype, hipStream_t s) {
+  const int64_t tpad = (ntok + KQ - 1) / KQ * KQ;
+  int ns = choose_splits(tpad, C, num_cus());
+  while (ns > 1 && (size_t)ns * (size_t)C * (size_t)lds * sizeof(float) > pcap) --ns;
+  int64_t span = (tpad + ns - 1) / ns;
+  span = (span + KQ - 1) / KQ * KQ;
+  ns = (int)((tpad + span - 1) / span);
+  float* P = ns > 1 ? Pbuf : nullptr;
+  const int nt = (int)((C + SM_T - 1) / SM_T);
+  const dim3 grid((unsigned)(nt * (nt + 1) / 2), (unsigned)ns);
+  SyrkTimer tm(s, C);
+#define CRBQ_SM_GO(T8_, F_) \
+  k_syrk16s<T8_, F_><<<grid, 256, 0, s>>>(X, ldx, ntok, tpad, (int)C, S, lds, nt, span, P)
+  if (dtype == CRBQ_F16) {
+    if (fast) CRBQ_SM_GO(h8_t, true); else CRBQ_SM_GO(h8_t, false);
+  } else {
+    if (fast) CRBQ_SM_GO(b8_t, true); else CRBQ_SM_GO(b8_t, false);
+  }
+#undef CRBQ_SM_GO
+  CRBQ_LAUNCH_CHECK();
+  tm.stop(s);
+  if (P) {
+    sum_splits(P, ns - 1, C, S, lds, s);
+    CRBQ_LAUNCH_CHECK();
+  }
+  return CRBQ_OK;
+}
+}  // namespace crbq
+
 extern "C" size_t crbq_hessian_workspace_size(int64_t ntok, int64_t C) {
   if (ntok <= 0 || C <= 0) return 0;
   if (C % crbq::ST == 0) {
@@ -1185,19 +1472,17 @@ extern "C" int crbq_hessian_accum(const void* X, int dtype, int64_t ntok, int64_
   if (ntok == 0) return CRBQ_OK;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == CRBQ_F32) {
-    const int nt = (int)((C + crbq::HT - 1) / crbq::HT);
-    const int64_t ntiles = (int64_t)nt * (nt + 1) / 2;
-    if (ntiles > 0x7fffffff) return CRBQ_ERR_ARG;
-    crbq::k_syrk32<<<(unsigned)ntiles, 256, 0, s>>>((const float*)X, ntok, ldx, (int)C, S,
-                                                    lds, nt);
-    CRBQ_LAUNCH_CHECK();
-    return CRBQ_OK;
+    return crbq::syrk32((const float*)X, ntok, ldx, C, S, lds, s);
   }
   if (dtype != CRBQ_F16 && dtype != CRBQ_BF16) return CRBQ_ERR_ARG;
   const int nt = (int)((C + crbq::ST - 1) / crbq::ST);
   const int64_t ntiles = (int64_t)nt * (nt + 1) / 2;
   if (ntiles > 0x7fffffff) return CRBQ_ERR_ARG;
   const bool fast = (C % 8 == 0) && (ldx % 8 == 0) && ((((uintptr_t)X) & 15) == 0);
+  const bool small = crbq::syrk16_small(ntok, C);
+  if (small && C % crbq::ST == 0)
+    return crbq::syrk16s((const uint16_t*)X, ldx, ntok, fast, C, S, lds, (float*)ws,
+                         ws ? ws_bytes : 0, dtype, s);
   if (fast && C % crbq::ST == 0 && ldx < ((int64_t)1 << 24)) {
     // token-major stages straight from X (no transposed copy); the
     // workspace holds the split partials and the control words
@@ -1213,6 +1498,12 @@ extern "C" int crbq_hessian_accum(const void* X, int dtype, int64_t ntok, int64_
     const size_t pcap = ws_bytes - pl.xt_bytes;
     for (int64_t t0 = 0; t0 < ntok; t0 += pl.tch) {
       const int64_t n = ntok - t0 < pl.tch ? ntok - t0 : pl.tch;
+      if (small) {                 // same passes and splits, no transposed copy
+        const int st = crbq::syrk16s((const uint16_t*)X + t0 * ldx, ldx, n, fast, C, S, lds,
+                                     Pbuf, pcap, dtype, s);
+        if (st) return st;
+        continue;
+      }
       const int64_t tpad = (n + crbq::KQ - 1) / crbq::KQ * crbq::KQ;
       const uint16_t* Xc = (const uint16_t*)X + t0 * ldx;
       const int64_t nw = (tpad / 64) * (pl.Cp / 64);
@@ -1230,6 +1521,9 @@ extern "C" int crbq_hessian_accum(const void* X, int dtype, int64_t ntok, int64_
     return CRBQ_OK;
   }
   // token-major path (workspace too small for the transposed copy)
+  if (small)
+    return crbq::syrk16s((const uint16_t*)X, ldx, ntok, fast, C, S, lds, (float*)ws,
+                         ws ? ws_bytes : 0, dtype, s);
   int ns = crbq::choose_splits(ntok, C, crbq::num_cus());
   // the partial buffers are laid out like S (row stride lds)
   while (ns > 1 && (!ws || (size_t)ns * (size_t)C * (size_t)lds * sizeof(float) > ws_bytes)) --ns;

@@ -380,6 +380,47 @@ def test_hessian_persistent_paced(dtype, T, C):
         assert torch.equal(torch.triu(S2), torch.triu(S))
 
 
+@pytest.mark.parametrize("T,C,ldx", [(1, 1, 1), (5, 33, 35), (37, 32, 36), (259, 65, 68),
+                                     (256, 2048, 2048), (131, 2049, 2051), (70, 2112, 2116)])
+def test_hessian_fp32_tiles(T, C, ldx):
+    """The fp32 SYRK at the edges of its 32 x 32 (up to 2048 channels) and 64
+    x 64 tiles and of its token chunks, aligned and not; against float64 (an
+    fp32 sum of T products, far below 1e-5), columns past C and the lower
+    triangle untouched."""
+    print(f"hessian fp32 T={T} C={C} ldx={ldx}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + C)
+    X = torch.randn(T, ldx, device=DEV, generator=g)[:, :C]
+    buf = torch.full((C, C + 3), 0.25, device=DEV)
+    S = buf[:, :C]
+    _k().hessian_accum(X, S)
+    torch.cuda.synchronize()
+    want = X.double().t() @ X.double() + 0.25
+    assert rel(torch.triu(S), torch.triu(want)) < 1e-5
+    assert torch.equal(torch.tril(S, -1), torch.tril(torch.full_like(S, 0.25), -1))
+    assert (buf[:, C:] == 0.25).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,C,ldx", [(1, 1, 1), (63, 63, 65), (65, 64, 64), (200, 72, 72),
+                                     (129, 130, 131), (6000, 136, 144)])
+def test_hessian_small_tiles(dtype, T, C, ldx):
+    """Few-tile calls run on 64 x 64 tiles straight from X: bitwise the sums
+    of the channel-major kernel on the same tokens and splits, at the edges
+    of the tiles and of the 64-token stages, aligned rows and not."""
+    print(f"hessian small {dtype} T={T} C={C} ldx={ldx}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + C)
+    X = torch.randn(T, ldx, device=DEV, generator=g).to(dtype)[:, :C]
+    S1 = torch.full((C, C), 0.5, device=DEV)
+    _k().hessian_accum(X, S1)
+    Xt = _k().hessian_cm_store(T, C, dtype, DEV)
+    _k().hessian_transpose(X, Xt, 0)
+    S2 = torch.full((C, C), 0.5, device=DEV)
+    _k().hessian_accum_cm(Xt, T, C, S2)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.triu(S1), torch.triu(S2))
+    assert (torch.tril(S1, -1) == torch.tril(torch.full_like(S1, 0.5), -1)).all()
+
+
 def test_hessian_matches_reference_add_batch():
     """Incremental rescale of bigptq.py:50-53 vs. one 2/n scaling."""
     print("hessian add_batch", flush=True)
