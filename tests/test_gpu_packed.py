@@ -51,6 +51,36 @@ def test_pack_matches_format_statement(R, C, dtype, n_odd):
     assert torch.equal(back.view(torch.int16).cpu(), Q.view(torch.int16).cpu())
 
 
+@pytest.mark.parametrize("R,C,pad,n_odd", [(1, 1, 0, 0), (3, 9, 1, 0), (5, 130, 3, 2),
+                                           (17, 136, 8, 1), (67, 257, 5, 9)])
+def test_pack_strided_edges(R, C, pad, n_odd):
+    """Block rows at the ends of a wavefront's four and rows and columns at the
+    ends of the matrix, weights and masks in rows of unaligned stride: pack
+    against the format statement, unpack (1 to 4 rows per thread) bit for bit
+    into an unaligned destination."""
+    print(f"pack edges {R}x{C} pad={pad} odd={n_odd}", flush=True)
+    from crb_amd import _lib
+    q, masks = structured(R, C, seed=R + C, n_odd=n_odd)
+    Qb = torch.zeros(R, C + pad, dtype=torch.float16, device=DEV)
+    Mb = torch.zeros(R, C + pad, dtype=torch.uint8, device=DEV)
+    Qb[:, :C], Mb[:, :C] = torch.from_numpy(q).to(DEV), torch.from_numpy(masks).to(DEV)
+    codes, lut, sal, ex = _k().pack(Qb[:, :C], Mb[:, :C])
+    rc, rl, rs, rex, st = pack_ref(q.view(np.uint16), masks)
+    assert st == 0
+    assert np.array_equal(codes.cpu().numpy(), rc)
+    assert np.array_equal(lut.cpu().view(torch.int16).numpy().view(np.uint16), rl)
+    assert np.array_equal(sal.cpu().numpy(), rs)
+    assert np.array_equal(ex.idx.cpu().numpy(), rex[0])
+    out = torch.full((R, C + pad + 1), 7.0, dtype=torch.float16, device=DEV)
+    lib = _lib.ready(out.device)
+    _lib.check(lib.crbq_unpack(codes.data_ptr(), codes.stride(0), lut.data_ptr(), sal.data_ptr(),
+                               ex.idx.data_ptr(), ex.val.data_ptr(), ex.idx.numel(), 1, R, C,
+                               out[:, 1:].data_ptr(), out.stride(0), _lib.stream_of(out)), "unpack")
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, 1:C + 1].view(torch.int16), Qb[:, :C].contiguous().view(torch.int16))
+    assert (out[:, :1] == 7).all() and (out[:, C + 1:] == 7).all()
+
+
 def test_pack_reports_structure_errors():
     print("pack errors", flush=True)
     from crb_amd._lib import CrbqError
