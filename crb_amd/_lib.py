@@ -53,6 +53,7 @@ class CrbqBlockTrace(ctypes.Structure):
 
 TRACE_BYTES = ctypes.sizeof(CrbqBlockTrace)
 NOALLOC_SCRATCH_BYTES = 80 << 20      # CRBQ_NOALLOC_SCRATCH_BYTES (include/crbq.h)
+LINEAR_MAX_EX = 256                   # CRBQ_LINEAR_MAX_EX
 ERR_TOO_LARGE = -5                    # CRBQ_ERR_TOO_LARGE
 ERR_CAPTURE = -6                      # CRBQ_ERR_CAPTURE
 
@@ -114,6 +115,9 @@ _SIGS = {
     "crbq_gemm_packed_workspace_size": (c_size, [c_i64, c_i64, c_i64]),
     "crbq_gemm_packed": (c_i32, [c_vp, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_i32, c_i64,
                                  c_i64, c_vp, c_i64, c_i64, c_vp, c_i64, c_vp, c_size, c_vp]),
+    "crbq_linear_packed": (c_i32, [c_vp, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_i32, c_i64,
+                                   c_i64, c_vp, c_i64, c_i64, c_vp, c_vp, c_i64, c_vp, c_size,
+                                   c_vp]),
 }
 
 _lock = threading.Lock()

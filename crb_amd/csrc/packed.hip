@@ -423,57 +423,6 @@ __global__ __launch_bounds__(256) void k_apply_ex(const int64_t* __restrict__ ex
 
 constexpr int GV_MAXVEC = 16;
 
-// The codes of pair p (elements 2p, 2p+1 of a lane's 8) are bits 4p..4p+1
-// and 4p+2..4p+3 of the 16-bit code word cw.  code_spread adds a copy of cw
-// 14 bits higher, so that pair p's two codes sit at bits 4p..4p+1 and
-// 4p+16..4p+17 for every p in 0..3, and one shift and one mask take them to
-// bits 0-1 and 16-17 (bits 16-31 of the argument are dropped).
-__device__ __forceinline__ uint32_t code_spread(uint32_t cw) {
-  return (cw & 0xffffu) | (cw << 14);
-}
-
-// Two weights (elements 2p, 2p+1 of a lane's 8) from the block's table L:
-// v_perm_b32 picks the 16-bit entries of codes (c_a, c_b) among the four
-// non-salient entries and among the four salient ones; selb (sal_sel of the
-// pair's two salient bits) takes each half from the salient or the
-// non-salient pick.  d is code_spread of the code word.
-__device__ __forceinline__ uint32_t decode_pair(uint32_t d, int p, uint4 L, uint32_t selb) {
-  const uint32_t t = (d >> (4 * p)) & 0x00030003u;     // c_a | c_b << 16
-  const uint32_t sel = t * 0x202u + 0x01000100u;
-  const uint32_t wn = __builtin_amdgcn_perm(L.y, L.x, sel);
-  const uint32_t ws = __builtin_amdgcn_perm(L.w, L.z, sel);
-  return __builtin_amdgcn_perm(ws, wn, selb);
-}
-
-// The final selector of pair q (columns 2q, 2q + 1) of a lane's 32 columns
-// from their salient bits sb: bytes 0-1 from the salient pick (perm source
-// bytes 4-7) if column 2q is salient, bytes 2-3 likewise for 2q + 1.
-__device__ __forceinline__ uint32_t sal_sel(uint32_t sb, int q) {
-  const uint32_t s2 = (sb >> (2 * q)) & 3u;
-  return 0x03020100u + (s2 & 1u) * 0x0404u + (s2 >> 1) * 0x04040000u;
-}
-
-// The 16 lanes of a DPP row (lanes 16 i .. 16 i + 15) decode the same 32
-// columns (one row of W each), so their selectors are the same: lane r of
-// the row builds pair r's (sal_sel(sb, r)) and the others read it with a
-// row broadcast (DPP row_newbcast), one move instead of the bit arithmetic.
-template <int Q>
-__device__ __forceinline__ uint32_t row_bcast_u32(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + Q, 0xf, 0xf, true);
-}
-__device__ __forceinline__ uint32_t pair_sel(uint32_t mine, int q) {   // q constant when unrolled
-  switch (q) {
-    case 0: return row_bcast_u32<0>(mine);   case 1: return row_bcast_u32<1>(mine);
-    case 2: return row_bcast_u32<2>(mine);   case 3: return row_bcast_u32<3>(mine);
-    case 4: return row_bcast_u32<4>(mine);   case 5: return row_bcast_u32<5>(mine);
-    case 6: return row_bcast_u32<6>(mine);   case 7: return row_bcast_u32<7>(mine);
-    case 8: return row_bcast_u32<8>(mine);   case 9: return row_bcast_u32<9>(mine);
-    case 10: return row_bcast_u32<10>(mine); case 11: return row_bcast_u32<11>(mine);
-    case 12: return row_bcast_u32<12>(mine); case 13: return row_bcast_u32<13>(mine);
-    case 14: return row_bcast_u32<14>(mine); default: return row_bcast_u32<15>(mine);
-  }
-}
-
 template <typename T8>
 __device__ __forceinline__ f4_t mfma_gv(T8 a, T8 b, f4_t c);
 template <>
@@ -485,26 +434,62 @@ __device__ __forceinline__ f4_t mfma_gv<b8_t>(b8_t a, b8_t b, f4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// What a fused linear layer adds to its fp32 sums before the one rounding to
+// the weights' dtype: the exceptions' delta * x (in list order) and the bias.
+struct PkEnd {
+  const uint16_t* bias;      // [R] in the weights' dtype, or NULL
+  const int64_t* ex_idx;
+  const float* ex_delta;
+  int n_ex;
+  bool bf16;
+};
+__device__ __forceinline__ uint32_t to_half_bits(float v, bool bf16) {
+  return bf16 ? (uint32_t)__builtin_bit_cast(unsigned short, (__bf16)v)
+              : (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)v);
+}
+// f(r, c, delta) for the exceptions with a row in [r_lo, r_hi), in list order;
+// called by whole wavefronts (64 list entries are tested at a time).
+template <typename F>
+__device__ __forceinline__ void for_ex(const PkEnd& e, int r_lo, int r_hi, int R, int C, F f) {
+  const int lane = threadIdx.x & 63;
+  if (r_hi > R) r_hi = R;
+  for (int base = 0; base < e.n_ex; base += 64) {
+    const bool in = base + lane < e.n_ex;
+    const int64_t i = in ? e.ex_idx[base + lane] : -1;
+    const float d = in ? e.ex_delta[base + lane] : 0.f;
+    const bool hit = i >= (int64_t)r_lo * C && i < (int64_t)r_hi * C;   // outside R x C: ignored
+    uint64_t m = __ballot(hit);
+    const int r = hit ? (int)(i / C) : 0, c = hit ? (int)(i - (int64_t)r * C) : 0;
+    while (m) {
+      const int j = __builtin_ctzll(m);
+      m &= m - 1;
+      f(__builtin_amdgcn_readlane(r, j), __builtin_amdgcn_readlane(c, j),
+        __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, d), j)));
+    }
+  }
+}
+
 // y[v][r] = sum_c W[r][c] x[v][c] for up to 16 vectors, W packed, x in the
 // weights' 16-bit dtype, fp32 sums, on v_mfma_f32_16x16x32.  A workgroup
 // takes 16 rows; its 16 wavefronts split the row's 128-column blocks into
 // contiguous ranges.  Per block, lane l takes the 32 contiguous columns
-// 32 (l >> 4) .. +31 of row l & 15 (8 bytes of codes, 4 of salient bits,
-// the row-block's table) and the same columns of vector l & 15 (64 bytes),
-// and feeds them to four MFMAs as 8-column slices: the MFMA sums over k in
-// any order as long as A and B agree, so the columns need not be in the
-// instruction's natural k order.  Decoding is the only per-weight vector
-// work whatever nvec.  The wavefronts' 16 x 16 partial products are
-// summed in LDS.
+// 32 (l >> 4) .. +31 of row l & 15 (8 bytes of codes and the row-block's
+// table) and the same columns of vector l & 15 (64 bytes), and feeds them to
+// four MFMAs as 8-column slices: the MFMA sums over k in any order as long
+// as A and B agree, so the columns need not be in the instruction's natural
+// k order.  The salient selectors are the same for every row: the workgroup
+// builds them once, in LDS, GV_SB blocks at a time.  The wavefronts' 16 x 16
+// partial products are summed in LDS.  END: the result is rounded to the
+// weights' dtype after bias and exceptions, else fp32.
 constexpr int GV_WAVES = 16;
+constexpr int GV_SB = 256;        // blocks of selectors in LDS (32 KB)
 
 template <typename T8>
-__device__ __forceinline__ void gv_block(const uint8_t* crow, const uint4* lrow,
-                                         const uint8_t* sal, const uint16_t* xv, int b, int kq,
-                                         int C, bool row_ok, bool vec_ok, f4_t& acc) {
+__device__ __forceinline__ void gv_block(const uint8_t* crow, const uint4* lrow, const uint32_t* S,
+                                         const uint16_t* xv, int b, int kq, int C, bool row_ok,
+                                         bool vec_ok, f4_t& acc) {
   const int c = b * PB + kq * 32;                // this lane's 32 columns
   const uint2 cw = row_ok ? *(const uint2*)(crow + b * 32 + kq * 8) : make_uint2(0u, 0u);
-  const uint32_t sb = *(const uint32_t*)(sal + (int64_t)b * 16 + kq * 4);
   const uint4 L = row_ok ? lrow[b] : make_uint4(0u, 0u, 0u, 0u);
   uint4 xs[4];
   if (c + 32 <= C) {                             // all blocks but a ragged last one
@@ -524,97 +509,131 @@ __device__ __forceinline__ void gv_block(const uint8_t* crow, const uint4* lrow,
                          h[6] | (h[7] << 16));
     }
   }
-  const uint32_t mine = sal_sel(sb, (int)(threadIdx.x & 15));
+  const uint4 s0 = *(const uint4*)(S + kq * 8), s1 = *(const uint4*)(S + kq * 8 + 4);
+  const Planes p = planes_of(L);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const uint32_t cws = code_spread((k < 2 ? cw.x : cw.y) >> (16 * (k & 1)));
-    uint4 a;
-    a.x = decode_pair(cws, 0, L, pair_sel(mine, 4 * k));
-    a.y = decode_pair(cws, 1, L, pair_sel(mine, 4 * k + 1));
-    a.z = decode_pair(cws, 2, L, pair_sel(mine, 4 * k + 2));
-    a.w = decode_pair(cws, 3, L, pair_sel(mine, 4 * k + 3));
-    acc = mfma_gv<T8>(__builtin_bit_cast(T8, a), __builtin_bit_cast(T8, xs[k]), acc);
+    const uint32_t w = (k < 2 ? cw.x : cw.y) >> (16 * (k & 1));
+    const uint4 sv = k < 2 ? s0 : s1;
+    const uint2 a0 = decode4(w & 0xffu, k & 1 ? sv.z : sv.x, p);
+    const uint2 a1 = decode4((w >> 8) & 0xffu, k & 1 ? sv.w : sv.y, p);
+    acc = mfma_gv<T8>(__builtin_bit_cast(T8, make_uint4(a0.x, a0.y, a1.x, a1.y)),
+                      __builtin_bit_cast(T8, xs[k]), acc);
   }
 }
 
-template <typename T8>
+template <typename T8, bool END>
 __global__ __launch_bounds__(64 * GV_WAVES) void k_gemv_packed(
     const uint8_t* __restrict__ codes, int64_t ldc, const uint16_t* __restrict__ lut,
     const uint8_t* __restrict__ sal, int R, int C, int nblk, const uint16_t* __restrict__ x,
-    int64_t ldx, int nvec, float* __restrict__ y, int64_t ldy) {
+    int64_t ldx, int nvec, void* __restrict__ y, int64_t ldy, PkEnd end) {
   __shared__ float red[GV_WAVES][16][17];
+  __shared__ __attribute__((aligned(16))) uint32_t Ss[GV_SB * 32];
   const int r0 = blockIdx.x * 16;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int row = r0 + (lane & 15), kq = lane >> 4, vec = lane & 15;
   const bool row_ok = row < R, vec_ok = vec < nvec;
-  const int b_beg = (int)((int64_t)nblk * wave / GV_WAVES);
-  const int b_end = (int)((int64_t)nblk * (wave + 1) / GV_WAVES);
   const uint8_t* crow = codes + (int64_t)(row_ok ? row : 0) * ldc;
   const uint4* lrow = (const uint4*)(lut + (int64_t)(row_ok ? row : 0) * nblk * 8);
   const uint16_t* xv = x + (int64_t)(vec_ok ? vec : 0) * ldx;
   f4_t acc = {0.f, 0.f, 0.f, 0.f};
-  int b = b_beg;
-  for (; b + 1 < b_end; b += 2) {
-    gv_block<T8>(crow, lrow, sal, xv, b, kq, C, row_ok, vec_ok, acc);
-    gv_block<T8>(crow, lrow, sal, xv, b + 1, kq, C, row_ok, vec_ok, acc);
+  for (int g = 0; g < nblk; g += GV_SB) {
+    const int n = min(GV_SB, nblk - g);
+    if (g) __syncthreads();                      // the last round's selectors are done with
+    for (int i = threadIdx.x; i < n * 32; i += 64 * GV_WAVES)
+      Ss[i] = sal_bytes(sal[(int64_t)g * 16 + (i >> 1)] >> (4 * (i & 1)));
+    __syncthreads();
+    const int b_end = (int)((int64_t)n * (wave + 1) / GV_WAVES);
+    int b = (int)((int64_t)n * wave / GV_WAVES);
+    for (; b + 1 < b_end; b += 2) {
+      gv_block<T8>(crow, lrow, Ss + b * 32, xv, g + b, kq, C, row_ok, vec_ok, acc);
+      gv_block<T8>(crow, lrow, Ss + b * 32 + 32, xv, g + b + 1, kq, C, row_ok, vec_ok, acc);
+    }
+    if (b < b_end) gv_block<T8>(crow, lrow, Ss + b * 32, xv, g + b, kq, C, row_ok, vec_ok, acc);
   }
-  if (b < b_end) gv_block<T8>(crow, lrow, sal, xv, b, kq, C, row_ok, vec_ok, acc);
   // acc[i] = partial y[vector lane & 15][row r0 + 4 (lane >> 4) + i]
 #pragma unroll
   for (int i = 0; i < 4; ++i) red[wave][4 * (lane >> 4) + i][lane & 15] = acc[i];
   __syncthreads();
   const int t = threadIdx.x;
   if (t < 256) {
-    const int rr = t >> 4, v = t & 15;
-    if (v < nvec && r0 + rr < R) {
-      float s0 = 0.f;
+    const int v = t >> 4, rr = t & 15;           // consecutive rows of one vector
+    float s0 = 0.f;
 #pragma unroll
-      for (int w = 0; w < GV_WAVES; ++w) s0 += red[w][rr][v];
-      y[(int64_t)v * ldy + r0 + rr] = s0;
+    for (int w = 0; w < GV_WAVES; ++w) s0 += red[w][rr][v];
+    const bool ok = v < nvec && r0 + rr < R;
+    if constexpr (END) {
+      for_ex(end, r0, r0 + 16, R, C, [&](int r, int c, float d) {
+        if (ok && r == r0 + rr) s0 += d * half_bits_to_float(x[(int64_t)v * ldx + c], end.bf16);
+      });
+      if (ok) {
+        if (end.bias) s0 += half_bits_to_float(end.bias[r0 + rr], end.bf16);
+        ((uint16_t*)y)[(int64_t)v * ldy + r0 + rr] = (uint16_t)to_half_bits(s0, end.bf16);
+      }
+    } else if (ok) {
+      ((float*)y)[(int64_t)v * ldy + r0 + rr] = s0;
     }
   }
 }
 
-// Y[t][r] = sum_c W[r][c] X[t][c] for many tokens (prefill), W packed:
-// the GEMV's decode, with each decoded fragment reused for a tile of
-// tokens.  A workgroup of GM_WAVES wavefronts covers 16 * GM_WAVES rows x
-// TT tokens (64, or 128 for more than 64 tokens); per 128-column block each wavefront decodes its 16 rows'
-// 128 columns (lane l: row l & 15, columns 32 (l >> 4) .. +31, four
-// 8-column MFMA slices) and multiplies them with every 16-token group of
-// the X tile, which the whole workgroup stages in LDS (rows padded to 136
-// halves so a 16-lane group's 16-byte reads of 16 tokens fall on disjoint
-// banks).  The X tile of the next block (with 64-token tiles also its codes,
-// salient bits and table) is loaded into registers while the current one is
-// used.  When row and token tiles alone would leave CUs idle
-// the block range is split over gridDim.z workgroups, each writing an fp32
-// partial [T][R] slice that k_gemm_packed_sum adds in split order.
-constexpr int GM_WAVES = 8;
-constexpr int GM_ROWS = 16 * GM_WAVES;
+// Y[t][r] = sum_c W[r][c] X[t][c] for many tokens (prefill), W packed: each
+// decoded fragment is reused for a tile of up to 16 TG tokens.  A workgroup
+// of GM_WAVES wavefronts covers GM_RT 16-row tiles per wavefront x tt tokens
+// (a multiple of 16, up to 16 TG: the tokens are split evenly); per
+// 128-column block each wavefront decodes its rows' 128 columns (lane l: row
+// l & 15 of each tile, columns 32 (l >> 4) .. +31, four 8-column MFMA slices)
+// and multiplies them with every 16-token group of the X tile, which the
+// whole workgroup stages in LDS (rows padded to 136 halves so a 16-lane
+// group's 16-byte reads of 16 tokens fall on disjoint banks) beside the
+// block's salient selectors.  With two row tiles an X fragment read from LDS
+// feeds two MFMAs, so that LDS and the matrix units are needed for the same
+// time; with one they wait for LDS twice as long (80 against 74 us at 4096 x
+// 16384 and 300 tokens).  When row and token tiles alone would leave CUs
+// idle the block range is split over gridDim.z workgroups, each writing an
+// fp32 partial [T][R] slice that k_gemm_packed_sum adds in split order.  END:
+// the result is rounded to the weights' dtype after bias and exceptions.
+// Counters at 4096 x 16384 and 256 tokens: MFMA busy 32 %, LDS 41 %, 246
+// vector instructions per wavefront and block, half of the wavefronts' time
+// in waits.  Codes and tables of four blocks at a time through LDS (whole
+// lines) measured no faster (85 us at 300 tokens, 34 against 22 at 17).
+constexpr int GM_WAVES = 8, GM_RT = 2;            // wavefronts, row tiles per wavefront
+constexpr int GM_ROWS = 16 * GM_RT * GM_WAVES;
 constexpr int GM_XP = PB + 8;                     // LDS pitch of an X tile row (halves)
 
-static inline int gemm_packed_tt(int64_t T) { return T > 64 ? 128 : 64; }
-
-template <typename T8, int GM_TT>
+template <typename T8, int TG, bool END>
 __global__ __launch_bounds__(64 * GM_WAVES) void k_gemm_packed(
     const uint8_t* __restrict__ codes, int64_t ldc, const uint16_t* __restrict__ lut,
     const uint8_t* __restrict__ sal, int R, int C, int nblk, const uint16_t* __restrict__ x,
-    int64_t ldx, int T, int bps, float* __restrict__ y, int64_t ldy) {
-  __shared__ __attribute__((aligned(16))) uint16_t Xs[2][GM_TT][GM_XP];
+    int64_t ldx, int T, int tt, int bps, void* __restrict__ y, int64_t ldy, PkEnd end) {
+  __shared__ __attribute__((aligned(16))) uint16_t Xs[2][16 * TG][GM_XP];
+  __shared__ __attribute__((aligned(16))) uint32_t Ss[2][32];
+  constexpr int RT = GM_RT;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int r0 = blockIdx.x * GM_ROWS, t0 = blockIdx.y * GM_TT;
+  const int r0 = (blockIdx.x * GM_WAVES + wave) * 16 * RT, t0 = blockIdx.y * tt;
   const int b_beg = blockIdx.z * bps, b_end = min(nblk, b_beg + bps);
-  const int row = r0 + wave * 16 + (lane & 15), kq = lane >> 4;
-  const bool row_ok = row < R;
-  const uint8_t* crow = codes + (int64_t)(row_ok ? row : 0) * ldc;
-  const uint4* lrow = (const uint4*)(lut + (int64_t)(row_ok ? row : 0) * nblk * 8);
+  const int kq = lane >> 4;
+  const int nt = min(tt, T - t0), ng = (nt + 15) / 16;
+  // rows past R read row 0: an MFMA output row depends only on its own
+  // weight row, and those rows are not stored
+  const uint8_t* crow[RT];
+  const uint4* lrow[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int row = r0 + 16 * i + (lane & 15);
+    crow[i] = codes + (int64_t)(row < R ? row : 0) * ldc + kq * 8;
+    lrow[i] = (const uint4*)(lut + (int64_t)(row < R ? row : 0) * nblk * 8);
+  }
   // X tile loader: thread -> (token xt, XPT 8-column chunks from xc)
-  constexpr int XPT = GM_TT * PB / 8 / (64 * GM_WAVES);     // 16-byte chunks per thread
+  constexpr int XPT = TG * 16 * PB / 8 / (64 * GM_WAVES);   // 16-byte chunks per thread
   constexpr int TPR = PB / 8 / XPT;                         // threads per token row
   const int xt = tid / TPR, xc = (tid % TPR) * XPT * 8;
-  const int tok = t0 + xt;
-  const bool tok_ok = tok < T;
-  const uint16_t* xrow = x + (int64_t)(tok_ok ? tok : 0) * ldx;
-  auto load_x = [&](int b, uint4 (&u)[XPT]) {
+  const bool tok_ok = xt < nt;
+  const uint16_t* xrow = x + (int64_t)(tok_ok ? t0 + xt : 0) * ldx;
+  uint4 u[XPT];
+  uint2 cw[RT];
+  uint4 L[RT];
+  uint32_t sb = 0;
+  auto load_x = [&](int b) {
     const int c = b * PB + xc;
     if (tok_ok && c + 8 * XPT <= C) {
 #pragma unroll
@@ -630,118 +649,249 @@ __global__ __launch_bounds__(64 * GM_WAVES) void k_gemm_packed(
       }
     }
   };
-  f4_t acc[GM_TT / 16];
+  auto load_codes = [&](int b) {                 // and tables and salient bits
 #pragma unroll
-  for (int g = 0; g < GM_TT / 16; ++g) acc[g] = f4_t{0.f, 0.f, 0.f, 0.f};
-  // With 64-token tiles a block's codes, salient bits and table are loaded
-  // with its X tile, one block ahead, so that the decode never waits on
-  // them (rows past R read row 0 through crow and lrow: an MFMA output row
-  // depends only on its own weight row, and those rows are not stored);
-  // 128-token tiles spread each decode over 8 token groups and load them
-  // after the barrier.
-  constexpr bool codes_ahead = GM_TT == 64;
-  uint4 u[XPT];
-  uint2 cwn = make_uint2(0u, 0u);
-  uint32_t sbn = 0u;
-  uint4 Ln = make_uint4(0u, 0u, 0u, 0u);
-  auto load_codes = [&](int b) {
-    cwn = *(const uint2*)(crow + b * 32 + kq * 8);
-    sbn = *(const uint32_t*)(sal + (int64_t)b * 16 + kq * 4);
-    Ln = lrow[b];
+    for (int i = 0; i < RT; ++i) {
+      cw[i] = *(const uint2*)(crow[i] + b * 32);
+      L[i] = lrow[i][b];
+    }
+    if (tid < 32) sb = sal[(int64_t)b * 16 + (tid >> 1)] >> (4 * (tid & 1));
+  };
+  f4_t acc[RT][TG];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int g = 0; g < TG; ++g) acc[i][g] = f4_t{0.f, 0.f, 0.f, 0.f};
+  // Fragment a[i][k] of a block from codes c, tables p and selectors s0, s1
+  T8 a[RT][4], an[RT][4];
+  auto decode = [&](T8& f, int k, uint2 c, const Planes& p, uint4 s0, uint4 s1) {
+    const uint32_t w = (k < 2 ? c.x : c.y) >> (16 * (k & 1));
+    const uint4 sv = k < 2 ? s0 : s1;
+    const uint2 a0 = decode4(w & 0xffu, k & 1 ? sv.z : sv.x, p);
+    const uint2 a1 = decode4((w >> 8) & 0xffu, k & 1 ? sv.w : sv.y, p);
+    f = __builtin_bit_cast(T8, make_uint4(a0.x, a0.y, a1.x, a1.y));
   };
   if (b_beg < b_end) {
-    if constexpr (codes_ahead) load_codes(b_beg);
-    load_x(b_beg, u);
+    load_codes(b_beg);
+    load_x(b_beg);
+    if (tid < 32) Ss[b_beg & 1][tid] = sal_bytes(sb);
+    __syncthreads();
+    const uint4 s0 = *(const uint4*)&Ss[b_beg & 1][kq * 8];
+    const uint4 s1 = *(const uint4*)&Ss[b_beg & 1][kq * 8 + 4];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      const Planes p = planes_of(L[i]);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) decode(a[i][k], k, cw[i], p, s0, s1);
+    }
+    load_codes(min(b_beg + 1, b_end - 1));
   }
+  // Block b: multiply its fragments while block b + 1's are decoded, a part
+  // with each token group (decoding at the top of a block, where the barrier
+  // has just lined the wavefronts up, left the matrix units idle meanwhile);
+  // X is loaded one block ahead, codes, tables and salient bits two.
   for (int b = b_beg; b < b_end; ++b) {
-    const int buf = (b - b_beg) & 1;
+    const int buf = b & 1;
 #pragma unroll
     for (int k = 0; k < XPT; ++k) *(uint4*)&Xs[buf][xt][xc + 8 * k] = u[k];
+    if (tid < 32) Ss[buf ^ 1][tid] = sal_bytes(sb);
+    uint2 cn[RT];
+    Planes p[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      cn[i] = cw[i];
+      p[i] = planes_of(L[i]);
+    }
     __syncthreads();
-    uint2 cw;
-    uint32_t sb;
-    uint4 L;
-    if constexpr (codes_ahead) {
-      cw = cwn;
-      sb = sbn;
-      L = Ln;
-      if (b + 1 < b_end) {
-        load_codes(b + 1);
-        load_x(b + 1, u);
+    load_x(min(b + 1, b_end - 1));
+    load_codes(min(b + 2, b_end - 1));
+    const uint4 s0 = *(const uint4*)&Ss[buf ^ 1][kq * 8];
+    const uint4 s1 = *(const uint4*)&Ss[buf ^ 1][kq * 8 + 4];
+    constexpr int PER = RT * 4 / TG > 0 ? RT * 4 / TG : 1;   // fragments decoded per group
+    auto part = [&](int g) {
+#pragma unroll
+      for (int q = 0; q < PER; ++q) {
+        const int f = g * PER + q;
+        if (f < RT * 4) decode(an[f >> 2][f & 3], f & 3, cn[f >> 2], p[f >> 2], s0, s1);
       }
-    } else {
-      if (b + 1 < b_end) load_x(b + 1, u);
-      cw = row_ok ? *(const uint2*)(crow + b * 32 + kq * 8) : make_uint2(0u, 0u);
-      sb = *(const uint32_t*)(sal + (int64_t)b * 16 + kq * 4);
-      L = row_ok ? lrow[b] : make_uint4(0u, 0u, 0u, 0u);
-    }
-    T8 a[4];
-    const uint32_t mine = sal_sel(sb, lane & 15);
+    };
+    // a group's X fragments are read while the group before it is multiplied
+    const uint16_t* xr = &Xs[buf][lane & 15][kq * 32];
+    T8 xf[2][4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t cws = code_spread((k < 2 ? cw.x : cw.y) >> (16 * (k & 1)));
-      uint4 q;
-      q.x = decode_pair(cws, 0, L, pair_sel(mine, 4 * k));
-      q.y = decode_pair(cws, 1, L, pair_sel(mine, 4 * k + 1));
-      q.z = decode_pair(cws, 2, L, pair_sel(mine, 4 * k + 2));
-      q.w = decode_pair(cws, 3, L, pair_sel(mine, 4 * k + 3));
-      a[k] = __builtin_bit_cast(T8, q);
+    for (int k = 0; k < 4; ++k) xf[0][k] = *(const T8*)(xr + 8 * k);
+#pragma unroll
+    for (int g = 0; g < TG; ++g) {
+      if (g < ng) {                               // uniform
+        if (g + 1 < TG) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            xf[(g + 1) & 1][k] = *(const T8*)(xr + (g + 1) * 16 * GM_XP + 8 * k);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < RT; ++i) acc[i][g] = mfma_gv<T8>(a[i][k], xf[g & 1][k], acc[i][g]);
+      }
+      part(g);
     }
 #pragma unroll
-    for (int g = 0; g < GM_TT / 16; ++g) {
-      if (t0 + g * 16 >= T) break;                // token groups past the end (uniform)
-      const uint16_t* xr = &Xs[buf][g * 16 + (lane & 15)][kq * 32];
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        acc[g] = mfma_gv<T8>(a[k], *(const T8*)(xr + 8 * k), acc[g]);
-    }
-    // the other buffer is written next; this one is only read again after
+      for (int k = 0; k < 4; ++k) a[i][k] = an[i][k];
+    // the other X buffer is written next; this one is only read again after
     // the following iteration's barrier
   }
-  // acc[g][i] = y[token t0 + 16 g + (lane & 15)][row r0 + 16 wave + 4 (lane >> 4) + i]
-  float* out = y + (size_t)blockIdx.z * (size_t)T * (size_t)ldy;
-  const int rb = r0 + wave * 16 + 4 * kq;
+  // acc[i][g][e] = y[token t0 + 16 g + (lane & 15)][row r0 + 16 i + 4 (lane >> 4) + e]
+  if constexpr (END) {
+    for_ex(end, r0, r0 + 16 * RT, R, C, [&](int r, int c, float d) {
 #pragma unroll
-  for (int g = 0; g < GM_TT / 16; ++g) {
-    const int t = t0 + g * 16 + (lane & 15);
-    if (t >= T) continue;
-    float* o = out + (int64_t)t * ldy + rb;
-    if (rb + 3 < R && ((((uintptr_t)o) & 15) == 0)) {
-      *(float4*)o = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
-    } else {
+      for (int g = 0; g < TG; ++g) {
+        const int t = g * 16 + (lane & 15);
+        if (t >= nt) continue;
+        const float dx = d * half_bits_to_float(x[(int64_t)(t0 + t) * ldx + c], end.bf16);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (rb + i < R) o[i] = acc[g][i];
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (r == r0 + 16 * i + 4 * kq + e) acc[i][g][e] += dx;
+      }
+    });
+  }
+  float* out = (float*)y + (size_t)blockIdx.z * (size_t)T * (size_t)ldy;
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int rb = r0 + 16 * i + 4 * kq;
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (END) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (end.bias && rb + e < R) bias[e] = half_bits_to_float(end.bias[rb + e], end.bf16);
+    }
+#pragma unroll
+    for (int g = 0; g < TG; ++g) {
+      const int t = g * 16 + (lane & 15);
+      if (t >= nt) continue;
+      if constexpr (END) {
+        uint16_t* o = (uint16_t*)y + (int64_t)(t0 + t) * ldy + rb;
+        uint32_t h[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = to_half_bits(acc[i][g][e] + bias[e], end.bf16);
+        if (rb + 3 < R && ((((uintptr_t)o) & 7) == 0)) {
+          *(uint2*)o = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (rb + e < R) o[e] = (uint16_t)h[e];
+        }
+      } else {
+        float* o = out + (int64_t)(t0 + t) * ldy + rb;
+        if (rb + 3 < R && ((((uintptr_t)o) & 15) == 0)) {
+          *(float4*)o = make_float4(acc[i][g][0], acc[i][g][1], acc[i][g][2], acc[i][g][3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (rb + e < R) o[e] = acc[i][g][e];
+        }
+      }
     }
   }
 }
 
-// y[t][r] = sum_s P[s][t][r] in split order
+// y[t][r] = sum_s P[s][t][r] in split order (P rows of R floats), 4 rows per
+// thread: grid (ceil(R / 1024), T).  END as above.
+template <bool END>
 __global__ __launch_bounds__(256) void k_gemm_packed_sum(const float* __restrict__ P, int ns,
-                                                         int T, int R, int64_t ldp,
-                                                         float* __restrict__ y, int64_t ldy) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)T * R) return;
-  const int t = (int)(idx / R), r = (int)(idx % R);
-  float v = 0.f;
-  for (int s = 0; s < ns; ++s) v += P[((int64_t)s * T + t) * ldp + r];
-  y[(int64_t)t * ldy + r] = v;
+                                                         int T, int R, int C,
+                                                         const uint16_t* __restrict__ x,
+                                                         int64_t ldx, void* __restrict__ y,
+                                                         int64_t ldy, PkEnd end) {
+  const int r = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const bool vec = (R & 3) == 0;
+  for (int t = blockIdx.y; t < T; t += gridDim.y) {
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    const float* p = P + (int64_t)t * R + r;
+    if (vec && r < R) {
+#pragma unroll 4
+      for (int s = 0; s < ns; ++s) {
+        const float4 q = *(const float4*)(p + (int64_t)s * T * R);
+        v[0] += q.x; v[1] += q.y; v[2] += q.z; v[3] += q.w;
+      }
+    } else {
+      for (int s = 0; s < ns; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (r + e < R) v[e] += p[(int64_t)s * T * R + e];
+    }
+    if constexpr (END) {
+      for_ex(end, 0, R, R, C, [&](int er, int c, float d) {
+        const float dx = d * half_bits_to_float(x[(int64_t)t * ldx + c], end.bf16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (er == r + e) v[e] += dx;
+      });
+      uint32_t h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (end.bias && r + e < R) v[e] += half_bits_to_float(end.bias[r + e], end.bf16);
+        h[e] = to_half_bits(v[e], end.bf16);
+      }
+      uint16_t* o = (uint16_t*)y + (int64_t)t * ldy + r;
+      if (r + 3 < R && ((((uintptr_t)o) & 7) == 0)) {
+        *(uint2*)o = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (r + e < R) o[e] = (uint16_t)h[e];
+      }
+    } else {
+      float* o = (float*)y + (int64_t)t * ldy + r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (r + e < R) o[e] = v[e];
+    }
+  }
 }
 
-// Split of the block range: as many splits as keep the workgroups within
-// 512 (two per CU of an MI355X, one round: a few workgroups past it would
-// run as a second round), at least 8 blocks per split; a function of the
-// shapes only, so the workspace size is known without a device.
-constexpr int GM_TARGET_WG = 512;
-static inline int gemm_packed_splits(int64_t R, int64_t C, int64_t T, int* bps) {
+// Launch shape of a packed product, a function of the shapes only so that
+// the workspace size is known without a device: 64-token tiles up to 64
+// tokens, else the tokens split evenly over tiles of up to 128, and the
+// number of column splits (of at least 2 blocks) with the least modelled
+// time: rounds of one workgroup per CU, each 5 us and 0.7 + 2.1 tt / 128 us a
+// block, and a sum launch of 3.5 us and the partials written and read at 4
+// TB/s.  Measured against
+// splits to fill the chip once, twice (us): 4096 x 16384 at 300 tokens 74 /
+// 83, at 768 167 / 151, 4096 x 4096 at 300 33 / 34, at 768 57 / 65; against no
+// split, 4096 x 1920 at 64 16 / 26, 1024 x 1024 at 128 18.5 / 24.  One-tile
+// products of up to 8 blocks take no workspace.
+struct GmPlan {
+  int tg, tt, ns, bps;
+  int64_t row_tiles, tok_tiles;
+};
+static inline GmPlan gemm_packed_plan(int64_t R, int64_t C, int64_t T) {
+  GmPlan p;
   const int64_t nblk = (C + PB - 1) / PB;
-  const int64_t tt = gemm_packed_tt(T);
-  const int64_t tiles = ((R + GM_ROWS - 1) / GM_ROWS) * ((T + tt - 1) / tt);
-  int64_t ns = GM_TARGET_WG / tiles;
-  ns = std::max<int64_t>(1, std::min<int64_t>(ns, nblk / 8));
-  const int64_t per = (nblk + ns - 1) / ns;
-  *bps = (int)per;
-  return (int)((nblk + per - 1) / per);
+  p.tg = T > 64 ? 8 : 4;
+  p.row_tiles = (R + GM_ROWS - 1) / GM_ROWS;
+  p.tok_tiles = (T + 16 * p.tg - 1) / (16 * p.tg);
+  p.tt = (int)(((T + p.tok_tiles - 1) / p.tok_tiles + 15) / 16 * 16);
+  p.tok_tiles = (T + p.tt - 1) / p.tt;
+  const int64_t tiles = p.row_tiles * p.tok_tiles;
+  const double block = 0.7 + 2.1 * p.tt / 128.0, slice = 8.0 * (double)T * (double)R / 4e6;
+  double best = 0.0;
+  p.ns = 0;
+  const int64_t most = tiles == 1 && nblk <= 8 ? 1 : std::max<int64_t>(1, nblk / 2);
+  for (int64_t ns = 1; ns == 1 || (ns <= most && tiles * ns <= 1024); ++ns) {
+    const int64_t per = (nblk + ns - 1) / ns, n = (nblk + per - 1) / per;
+    const double t = (double)((tiles * n + 255) / 256) * (5.0 + block * (double)per) +
+                     (n > 1 ? 3.5 + slice * (double)n : 0.0);
+    if (p.ns == 0 || t < best) {
+      best = t;
+      p.ns = (int)n;
+      p.bps = (int)per;
+    }
+  }
+  return p;
 }
 
 }  // namespace crbq
@@ -805,46 +955,11 @@ static int apply_ex(const int64_t* ex_idx, const float* ex_delta, int64_t n_ex, 
   return CRBQ_OK;
 }
 
-extern "C" int crbq_gemv_packed(const uint8_t* codes, int64_t ldc, const void* lut,
-                                const uint8_t* sal, const int64_t* ex_idx,
-                                const float* ex_delta, int64_t n_ex, int dtype, int64_t R,
-                                int64_t C, const void* x, int64_t ldx, int nvec, float* y,
-                                int64_t ldy, void* stream) {
-  if (!codes || !lut || !sal || !x || !y) return CRBQ_ERR_ARG;
-  if (n_ex < 0 || (n_ex > 0 && (!ex_idx || !ex_delta))) return CRBQ_ERR_ARG;
-  if (dtype != CRBQ_F16 && dtype != CRBQ_BF16) return CRBQ_ERR_ARG;
-  if (R <= 0 || C <= 0 || R > 0x7fffffff || C > 0x7fffffff) return CRBQ_ERR_ARG;
-  if (nvec < 1 || nvec > crbq::GV_MAXVEC || ldx < C || ldy < R) return CRBQ_ERR_ARG;
-  const int64_t nblk = (C + crbq::PB - 1) / crbq::PB;
-  if (ldc < nblk * 32 || (ldc & 7) || (ldx & 7) || (((uintptr_t)x) & 15) ||
-      (((uintptr_t)lut) & 15) || (((uintptr_t)codes) & 7) || (((uintptr_t)sal) & 3))
-    return CRBQ_ERR_ARG;
-  const unsigned grid = (unsigned)((R + 15) / 16);
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype == CRBQ_BF16)
-    crbq::k_gemv_packed<b8_t><<<grid, 64 * crbq::GV_WAVES, 0, s>>>(
-        codes, ldc, (const uint16_t*)lut, sal, (int)R, (int)C, (int)nblk, (const uint16_t*)x,
-        ldx, nvec, y, ldy);
-  else
-    crbq::k_gemv_packed<h8_t><<<grid, 64 * crbq::GV_WAVES, 0, s>>>(
-        codes, ldc, (const uint16_t*)lut, sal, (int)R, (int)C, (int)nblk, (const uint16_t*)x,
-        ldx, nvec, y, ldy);
-  CRBQ_LAUNCH_CHECK();
-  return apply_ex(ex_idx, ex_delta, n_ex, R, C, x, ldx, dtype, nvec, y, ldy, s);
-}
-
-extern "C" size_t crbq_gemm_packed_workspace_size(int64_t R, int64_t C, int64_t ntok) {
-  if (R <= 0 || C <= 0 || ntok <= 0) return 0;
-  int bps = 0;
-  const int ns = crbq::gemm_packed_splits(R, C, ntok, &bps);
-  return ns > 1 ? (size_t)ns * (size_t)ntok * (size_t)R * sizeof(float) : 0;
-}
-
-extern "C" int crbq_gemm_packed(const uint8_t* codes, int64_t ldc, const void* lut,
-                                const uint8_t* sal, const int64_t* ex_idx,
-                                const float* ex_delta, int64_t n_ex, int dtype, int64_t R,
-                                int64_t C, const void* x, int64_t ldx, int64_t ntok, float* y,
-                                int64_t ldy, void* ws, size_t ws_bytes, void* stream) {
+// Argument checks the packed products share.
+static int packed_check(const uint8_t* codes, int64_t ldc, const void* lut, const uint8_t* sal,
+                        const int64_t* ex_idx, const float* ex_delta, int64_t n_ex, int dtype,
+                        int64_t R, int64_t C, const void* x, int64_t ldx, int64_t ntok,
+                        const void* y, int64_t ldy) {
   if (!codes || !lut || !sal || !x || !y) return CRBQ_ERR_ARG;
   if (n_ex < 0 || (n_ex > 0 && (!ex_idx || !ex_delta))) return CRBQ_ERR_ARG;
   if (dtype != CRBQ_F16 && dtype != CRBQ_BF16) return CRBQ_ERR_ARG;
@@ -855,33 +970,118 @@ extern "C" int crbq_gemm_packed(const uint8_t* codes, int64_t ldc, const void* l
   if (ldc < nblk * 32 || (ldc & 7) || (ldx & 7) || (((uintptr_t)x) & 15) ||
       (((uintptr_t)lut) & 15) || (((uintptr_t)codes) & 7) || (((uintptr_t)sal) & 3))
     return CRBQ_ERR_ARG;
-  int bps = 0;
-  const int ns = crbq::gemm_packed_splits(R, C, ntok, &bps);
-  const size_t need = ns > 1 ? (size_t)ns * (size_t)ntok * (size_t)R * sizeof(float) : 0;
+  return CRBQ_OK;
+}
+
+template <bool END>
+static int gemv_go(const uint8_t* codes, int64_t ldc, const void* lut, const uint8_t* sal,
+                   int dtype, int64_t R, int64_t C, const void* x, int64_t ldx, int nvec, void* y,
+                   int64_t ldy, const crbq::PkEnd& end, hipStream_t s) {
+  const int nblk = (int)((C + crbq::PB - 1) / crbq::PB);
+  const unsigned grid = (unsigned)((R + 15) / 16);
+  if (dtype == CRBQ_BF16)
+    crbq::k_gemv_packed<b8_t, END><<<grid, 64 * crbq::GV_WAVES, 0, s>>>(
+        codes, ldc, (const uint16_t*)lut, sal, (int)R, (int)C, nblk, (const uint16_t*)x, ldx,
+        nvec, y, ldy, end);
+  else
+    crbq::k_gemv_packed<h8_t, END><<<grid, 64 * crbq::GV_WAVES, 0, s>>>(
+        codes, ldc, (const uint16_t*)lut, sal, (int)R, (int)C, nblk, (const uint16_t*)x, ldx,
+        nvec, y, ldy, end);
+  CRBQ_LAUNCH_CHECK();
+  return CRBQ_OK;
+}
+
+static size_t gemm_ws_bytes(const crbq::GmPlan& p, int64_t R, int64_t T) {
+  return p.ns > 1 ? (size_t)p.ns * (size_t)T * (size_t)R * sizeof(float) : 0;
+}
+
+// END: y is [ntok][ldy] in the weights' dtype, else fp32.
+template <bool END>
+static int gemm_go(const uint8_t* codes, int64_t ldc, const void* lut, const uint8_t* sal,
+                   int dtype, int64_t R, int64_t C, const void* x, int64_t ldx, int64_t ntok,
+                   void* y, int64_t ldy, const crbq::PkEnd& end, void* ws, size_t ws_bytes,
+                   hipStream_t s) {
+  const int nblk = (int)((C + crbq::PB - 1) / crbq::PB);
+  const crbq::GmPlan p = crbq::gemm_packed_plan(R, C, ntok);
+  const size_t need = gemm_ws_bytes(p, R, ntok);
   if (need && (!ws || ws_bytes < need)) return CRBQ_ERR_WORKSPACE;
-  float* out = ns > 1 ? (float*)ws : y;
-  const int64_t ldo = ns > 1 ? R : ldy;
-  const int tt = crbq::gemm_packed_tt(ntok);
-  dim3 grid((unsigned)((R + crbq::GM_ROWS - 1) / crbq::GM_ROWS),
-            (unsigned)((ntok + tt - 1) / tt), (unsigned)ns);
-  if (grid.y > 65535) return CRBQ_ERR_ARG;
-  hipStream_t s = (hipStream_t)stream;
-#define CRBQ_GM_LAUNCH(T8, TT)                                                                  \
-  crbq::k_gemm_packed<T8, TT><<<grid, 64 * crbq::GM_WAVES, 0, s>>>(                             \
-      codes, ldc, (const uint16_t*)lut, sal, (int)R, (int)C, (int)nblk, (const uint16_t*)x,     \
-      ldx, (int)ntok, bps, out, ldo)
-  if (dtype == CRBQ_BF16) {
-    if (tt == 128) CRBQ_GM_LAUNCH(b8_t, 128); else CRBQ_GM_LAUNCH(b8_t, 64);
+  if (p.tok_tiles > 65535) return CRBQ_ERR_ARG;
+  const dim3 grid((unsigned)p.row_tiles, (unsigned)p.tok_tiles, (unsigned)p.ns);
+  const bool split = p.ns > 1;
+  void* out = split ? ws : y;
+  const int64_t ldo = split ? R : ldy;
+#define CRBQ_GM_LAUNCH(T8, TG, E)                                                               \
+  crbq::k_gemm_packed<T8, TG, E><<<grid, 64 * crbq::GM_WAVES, 0, s>>>(                          \
+      codes, ldc, (const uint16_t*)lut, sal, (int)R, (int)C, nblk, (const uint16_t*)x, ldx,     \
+      (int)ntok, p.tt, p.bps, out, ldo, end)
+#define CRBQ_GM_TILE(T8, E) \
+  do { if (p.tg == 8) CRBQ_GM_LAUNCH(T8, 8, E); else CRBQ_GM_LAUNCH(T8, 4, E); } while (0)
+  if (END && !split) {
+    if (dtype == CRBQ_BF16) CRBQ_GM_TILE(b8_t, true); else CRBQ_GM_TILE(h8_t, true);
   } else {
-    if (tt == 128) CRBQ_GM_LAUNCH(h8_t, 128); else CRBQ_GM_LAUNCH(h8_t, 64);
+    if (dtype == CRBQ_BF16) CRBQ_GM_TILE(b8_t, false); else CRBQ_GM_TILE(h8_t, false);
   }
+#undef CRBQ_GM_TILE
 #undef CRBQ_GM_LAUNCH
   CRBQ_LAUNCH_CHECK();
-  if (ns > 1) {
-    const int64_t n = ntok * R;
-    crbq::k_gemm_packed_sum<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
-        out, ns, (int)ntok, (int)R, R, y, ldy);
+  if (split) {
+    const dim3 sg((unsigned)((R + 1023) / 1024), (unsigned)std::min<int64_t>(ntok, 65535));
+    crbq::k_gemm_packed_sum<END><<<sg, 256, 0, s>>>((const float*)ws, p.ns, (int)ntok, (int)R,
+                                                    (int)C, (const uint16_t*)x, ldx, y, ldy, end);
     CRBQ_LAUNCH_CHECK();
   }
+  return CRBQ_OK;
+}
+
+extern "C" int crbq_gemv_packed(const uint8_t* codes, int64_t ldc, const void* lut,
+                                const uint8_t* sal, const int64_t* ex_idx,
+                                const float* ex_delta, int64_t n_ex, int dtype, int64_t R,
+                                int64_t C, const void* x, int64_t ldx, int nvec, float* y,
+                                int64_t ldy, void* stream) {
+  if (nvec < 1 || nvec > crbq::GV_MAXVEC) return CRBQ_ERR_ARG;
+  int st = packed_check(codes, ldc, lut, sal, ex_idx, ex_delta, n_ex, dtype, R, C, x, ldx, nvec,
+                        y, ldy);
+  if (st) return st;
+  hipStream_t s = (hipStream_t)stream;
+  st = gemv_go<false>(codes, ldc, lut, sal, dtype, R, C, x, ldx, nvec, y, ldy, crbq::PkEnd{}, s);
+  if (st) return st;
+  return apply_ex(ex_idx, ex_delta, n_ex, R, C, x, ldx, dtype, nvec, y, ldy, s);
+}
+
+extern "C" size_t crbq_gemm_packed_workspace_size(int64_t R, int64_t C, int64_t ntok) {
+  if (R <= 0 || C <= 0 || ntok <= 0) return 0;
+  return gemm_ws_bytes(crbq::gemm_packed_plan(R, C, ntok), R, ntok);
+}
+
+extern "C" int crbq_gemm_packed(const uint8_t* codes, int64_t ldc, const void* lut,
+                                const uint8_t* sal, const int64_t* ex_idx,
+                                const float* ex_delta, int64_t n_ex, int dtype, int64_t R,
+                                int64_t C, const void* x, int64_t ldx, int64_t ntok, float* y,
+                                int64_t ldy, void* ws, size_t ws_bytes, void* stream) {
+  int st = packed_check(codes, ldc, lut, sal, ex_idx, ex_delta, n_ex, dtype, R, C, x, ldx, ntok,
+                        y, ldy);
+  if (st) return st;
+  hipStream_t s = (hipStream_t)stream;
+  st = gemm_go<false>(codes, ldc, lut, sal, dtype, R, C, x, ldx, ntok, y, ldy, crbq::PkEnd{}, ws,
+                      ws_bytes, s);
+  if (st) return st;
   return apply_ex(ex_idx, ex_delta, n_ex, R, C, x, ldx, dtype, ntok, y, ldy, s);
+}
+
+extern "C" int crbq_linear_packed(const uint8_t* codes, int64_t ldc, const void* lut,
+                                  const uint8_t* sal, const int64_t* ex_idx,
+                                  const float* ex_delta, int64_t n_ex, int dtype, int64_t R,
+                                  int64_t C, const void* x, int64_t ldx, int64_t ntok,
+                                  const void* bias, void* y, int64_t ldy, void* ws,
+                                  size_t ws_bytes, void* stream) {
+  const int st = packed_check(codes, ldc, lut, sal, ex_idx, ex_delta, n_ex, dtype, R, C, x, ldx,
+                              ntok, y, ldy);
+  if (st) return st;
+  if (n_ex > CRBQ_LINEAR_MAX_EX) return CRBQ_ERR_ARG;
+  const crbq::PkEnd end{(const uint16_t*)bias, ex_idx, ex_delta, (int)n_ex, dtype == CRBQ_BF16};
+  hipStream_t s = (hipStream_t)stream;
+  if (ntok <= crbq::GV_MAXVEC)
+    return gemv_go<true>(codes, ldc, lut, sal, dtype, R, C, x, ldx, (int)ntok, y, ldy, end, s);
+  return gemm_go<true>(codes, ldc, lut, sal, dtype, R, C, x, ldx, ntok, y, ldy, end, ws, ws_bytes,
+                       s);
 }

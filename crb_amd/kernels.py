@@ -499,3 +499,29 @@ def gemm_packed(codes: torch.Tensor, lut: torch.Tensor, sal: torch.Tensor, C: in
                                ws.data_ptr(), nws, stream_of(y)),
           "crbq_gemm_packed")
     return y
+
+
+def linear_packed(codes: torch.Tensor, lut: torch.Tensor, sal: torch.Tensor, C: int,
+                  x: torch.Tensor, bias: torch.Tensor | None = None,
+                  ex: PackedEx | None = None) -> torch.Tensor:
+    """y [T, R] in the weights' dtype = x [T, C] @ W^T + bias for the packed W:
+    the GEMV up to 16 tokens, the GEMM above, bias (in the weights' dtype) and
+    exceptions added to the fp32 sums before the one rounding.  At most
+    LINEAR_MAX_EX exceptions."""
+    _dev_check(codes, lut, sal, x, bias)
+    x = _packed_x(x, lut, C, "linear_packed")
+    T, R = x.shape[0], codes.shape[0]
+    if bias is not None and (bias.dtype != lut.dtype or tuple(bias.shape) != (R,)
+                             or bias.stride(0) != 1):
+        raise _lib.CrbqError("linear_packed takes a contiguous [R] bias in the weights' dtype")
+    y = torch.empty((T, R), dtype=lut.dtype, device=x.device)
+    lib = _lib.ready(x.device)
+    nws = int(lib.crbq_gemm_packed_workspace_size(R, C, T)) if T > 16 else 0
+    ws = _ws(nws, x.device) if nws else None
+    ei, _, ed, n = _ex_args(ex, x.device, lut.dtype)
+    check(lib.crbq_linear_packed(codes.data_ptr(), codes.stride(0), lut.data_ptr(),
+                                 sal.data_ptr(), ei, ed, n, _lib.DTYPES[lut.dtype], R, C,
+                                 x.data_ptr(), x.stride(0), T, ptr(bias), y.data_ptr(),
+                                 y.stride(0), ptr(ws), nws, stream_of(y)),
+          "crbq_linear_packed")
+    return y

@@ -6,8 +6,8 @@ The reference stores a quantized layer as fake-quantized fp16/bf16 weights
 row, one salient-column bitmap per block; the format is described in
 include/crbq.h) and multiplies with them directly: up to 16 tokens per call
 through the packed GEMV (MFMA on weights decoded in registers), up to 768
-through the packed GEMM (each decoded fragment reused for 64 or 128 tokens),
-and larger batches, where the product is compute-bound, by unpacking into a
+through the packed GEMM (each decoded fragment reused for up to 128 tokens),
+with bias and rounding in the same kernels, and larger batches, where the product is compute-bound, by unpacking into a
 temporary dense weight for the dense GEMM.  The limits are the measured
 crossovers on MI355X (4096 x 16384 and 16384 x 4096 fp16 layers).
 """
@@ -18,6 +18,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import kernels
+from ._lib import LINEAR_MAX_EX
 
 GEMV_MAX_TOKENS = 16
 GEMM_MAX_TOKENS = 768
@@ -60,10 +61,20 @@ class PackedLinear(nn.Module):
         """The dense quantized weight (bit-identical to what was packed)."""
         return kernels.unpack(self.codes, self.lut, self.sal, self.in_features, self.ex)
 
+    def _fused(self, x: torch.Tensor) -> bool:
+        """Product, exceptions, bias and rounding in one kernel: activations
+        and bias in the weights' dtype and few exceptions."""
+        b = self.bias
+        return (x.dtype == self.lut.dtype and self.ex_idx.numel() <= LINEAR_MAX_EX
+                and (b is None or (b.dtype == x.dtype and b.is_contiguous())))
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
-        if x2.shape[0] <= GEMM_MAX_TOKENS:
+        if x2.shape[0] <= GEMM_MAX_TOKENS and self._fused(x):
+            y = kernels.linear_packed(self.codes, self.lut, self.sal, self.in_features, x2,
+                                      self.bias, self.ex)
+        elif x2.shape[0] <= GEMM_MAX_TOKENS:
             mm = kernels.gemv_packed if x2.shape[0] <= GEMV_MAX_TOKENS else kernels.gemm_packed
             y = mm(self.codes, self.lut, self.sal, self.in_features, x2, self.ex)
             y = y.to(x.dtype)

@@ -323,10 +323,9 @@ int crbq_gemv_packed(const uint8_t* codes, int64_t ldc, const void* lut,
  * count; meant for prefill batches above the GEMV's 16), X in the weights'
  * dtype (ldx multiple of 8, 16-byte aligned), fp32 Y [ntok][ldy], the
  * exceptions added as in the GEMV.  Each decoded weight fragment is reused
- * for 64 tokens (128 above 64).  When the shapes give 256 or fewer row x
- * token tiles (128 rows each) the column blocks are split over workgroups
- * (floor(512 / tiles) splits of at least 8 blocks) whose fp32 partials go to
- * the workspace and are summed in split order (deterministic);
+ * for up to 128 tokens.  When the shapes give few row x token tiles the
+ * column blocks are split over workgroups whose fp32 partials go to the
+ * workspace and are summed in split order (deterministic);
  * crbq_gemm_packed_workspace_size(R, C, ntok) bytes (0 when there is no
  * split) depend on the shapes only. */
 size_t crbq_gemm_packed_workspace_size(int64_t R, int64_t C, int64_t ntok);
@@ -335,6 +334,20 @@ int crbq_gemm_packed(const uint8_t* codes, int64_t ldc, const void* lut,
                      int64_t n_ex, int dtype, int64_t R, int64_t C, const void* x,
                      int64_t ldx, int64_t ntok, float* y, int64_t ldy, void* ws,
                      size_t ws_bytes, void* stream);
+
+/* crbq_linear_packed: a packed linear layer in one go, y[t][r] = round(
+ * sum_c W[r][c] x[t][c] + exceptions + bias[r]) in the weights' dtype: the
+ * GEMV (up to 16 tokens) or the GEMM (above) with bias (the weights' dtype,
+ * or NULL) and exceptions added to the fp32 sums before the one rounding.
+ * y [ntok][ldy] 16-bit; at most CRBQ_LINEAR_MAX_EX exceptions (else
+ * CRBQ_ERR_ARG).  Workspace: none up to 16 tokens, above
+ * crbq_gemm_packed_workspace_size. */
+#define CRBQ_LINEAR_MAX_EX 256
+int crbq_linear_packed(const uint8_t* codes, int64_t ldc, const void* lut, const uint8_t* sal,
+                       const int64_t* ex_idx, const float* ex_delta, int64_t n_ex, int dtype,
+                       int64_t R, int64_t C, const void* x, int64_t ldx, int64_t ntok,
+                       const void* bias, void* y, int64_t ldy, void* ws, size_t ws_bytes,
+                       void* stream);
 
 #ifdef __cplusplus
 }

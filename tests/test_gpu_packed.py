@@ -240,3 +240,33 @@ def test_stack_pack_option():
         x = samples[:1, :5]
         la_, lb_ = a(x).logits.float(), b(x).logits.float()
     assert torch.allclose(la_, lb_, rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("R,C,T,dtype,bias,n_odd", [
+    (17, 136, 1, torch.float16, True, 0), (33, 300, 16, torch.bfloat16, True, 3),
+    (256, 1024, 64, torch.float16, True, 70),          # one launch, two list rounds
+    (300, 1920, 17, torch.float16, False, 4),          # split sums
+    (257, 640, 65, torch.bfloat16, True, 5), (250, 520, 129, torch.float16, True, 2),
+    (515, 2049, 300, torch.bfloat16, True, 9), (1, 9, 3, torch.float16, True, 0)])
+def test_linear_packed_against_float64(R, C, T, dtype, bias, n_odd):
+    """crbq_linear_packed (sums, exceptions, bias, one rounding) against
+    float64: half an ulp of the 16-bit result (2^-11 or 2^-8 relative) plus the
+    GEMV's fp32 bar; columns past R untouched; PackedLinear takes it for
+    activations and bias of the weights' dtype."""
+    print(f"linear packed {R}x{C} T={T} {dtype} odd={n_odd}", flush=True)
+    from crb_amd.packed import PackedLinear
+    q, masks = structured(R, C, seed=3 * R + C, n_odd=n_odd)
+    Q = _q16(q, dtype)
+    codes, lut, sal, ex = _k().pack(Q, torch.from_numpy(masks).to(DEV))
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, C + 16, generator=g).to(dtype).to(DEV)[:, :C]
+    b = torch.randn(R, generator=g).to(dtype).to(DEV) if bias else None
+    y = _k().linear_packed(codes, lut, sal, C, x, b, ex)
+    assert y.dtype == dtype and y.shape == (T, R)
+    x64, W64 = x.double().cpu(), Q.double().cpu()
+    ref = x64 @ W64.t() + (b.double().cpu() if bias else 0.0)
+    scale = x64.abs() @ W64.abs().t() + (b.double().cpu().abs() if bias else 0.0)
+    half_ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    err = (y.double().cpu() - ref).abs()
+    assert (err <= half_ulp * ref.abs() + 1.1e-5 * scale + 2.0 ** -25).all()
+    assert torch.equal(PackedLinear(codes, lut, sal, C, b, ex)(x), y)
