@@ -41,10 +41,8 @@ constexpr int NQ = 81;       // percentiles linspace(0.10, 0.90, 81)
 constexpr int NT = 2 * NQ;   // order statistics needed (lo, hi per percentile)
 constexpr int NCMAX = 128;   // widest block
 constexpr int UPMAX = 64;    // largest supported up_lim
-#ifndef CRBQ_Q_RPW
-#define CRBQ_Q_RPW 32
-#endif
-constexpr int Q_RPW = CRBQ_Q_RPW;   // rows per workgroup in the quantile passes
+constexpr int Q_RPW = 32;    // rows per workgroup in the quantile passes
+constexpr int Q_RPW_S = 8;   // with few rows, so that they spread over the CUs
 #ifndef CRBQ_CS_MAXWG
 #define CRBQ_CS_MAXWG 128
 #endif
@@ -324,9 +322,8 @@ struct ParA {           // a group's fp32 parameters for the residual pass
 // workgroup's rows (row r0 + i / nc, column i % nc).  Every load of W is
 // issued before any is used, so the loads overlap instead of each waiting
 // out a memory latency.
-constexpr int QE = Q_RPW * NCMAX / 256;
-static_assert(QE * 256 == Q_RPW * NCMAX, "quantile pass geometry");
-
+// RPW: rows per workgroup.
+template <int QE>
 __device__ __forceinline__ void q_load(const float* __restrict__ W, int64_t ldw, int r0, int r1,
                                        int nc, float (&w)[QE], int (&col)[QE]) {
   const int n = (r1 - r0) * nc;
@@ -354,6 +351,7 @@ __device__ __forceinline__ void q_cols(const float* __restrict__ U, int64_t ldu,
 }
 
 // Level-1: histogram of bits [31:20] of the (non-negative) float pattern.
+template <int RPW>
 __global__ __launch_bounds__(256) void k_qpass1(
     SegSearch seg, int64_t ldw, int R, int nc, int64_t ldu,
     int metric) {
@@ -364,10 +362,11 @@ __global__ __launch_bounds__(256) void k_qpass1(
   __shared__ float d2s[NCMAX];
   __shared__ int rk[NCMAX];
   const int tid = threadIdx.x;
-  const int r0 = blockIdx.x * Q_RPW, r1 = min(R, r0 + Q_RPW);
+  constexpr int QE = RPW * NCMAX / 256;
+  const int r0 = blockIdx.x * RPW, r1 = min(R, r0 + RPW);
   float w[QE];
   int col[QE];
-  q_load(W, ldw, r0, r1, nc, w, col);
+  q_load<QE>(W, ldw, r0, r1, nc, w, col);
   for (int i = tid; i < H1; i += 256) lh[i] = 0u;
   const int istar = s.ctrl->istar;
   q_cols(U, ldu, nc, s, rk, d2s);
@@ -457,6 +456,7 @@ __device__ __forceinline__ int find_bin(const uint32_t* cum, uint32_t r) {
 // one global atomic per list, and writes the elements' bit patterns (the
 // order inside a list does not matter to the selection).  The list counters
 // are cleared by k_colscore.
+template <int RPW>
 __global__ __launch_bounds__(256) void k_qlist(
     SegSearch seg, int64_t ldw, int R, int nc, int64_t ldu,
     int metric) {
@@ -473,11 +473,12 @@ __global__ __launch_bounds__(256) void k_qlist(
   __shared__ int loff[NT];
   __shared__ int bins[NT];
   const int tid = threadIdx.x;
-  const int r0 = blockIdx.x * Q_RPW, r1 = min(R, r0 + Q_RPW);
+  constexpr int QE = RPW * NCMAX / 256;
+  const int r0 = blockIdx.x * RPW, r1 = min(R, r0 + RPW);
   const int64_t n = (int64_t)R * nc;
   float w[QE];
   int col[QE];
-  q_load(W, ldw, r0, r1, nc, w, col);
+  q_load<QE>(W, ldw, r0, r1, nc, w, col);
   const int istar = s.ctrl->istar;
   q_cols(U, ldu, nc, s, rk, d2s);
   for (int i = tid; i < H1; i += 256) lead[i] = NONE;
@@ -861,9 +862,10 @@ __device__ __forceinline__ void wave_prefix(SortedRow& r, float x0, float x1, in
 // fp64 prefix sums of v and v^2; then the workgroup's (row, candidate k)
 // pairs over all its lanes, each two binary searches per group and range
 // sums (group_err1); the last workgroup takes k* = first strict minimum.
+// rpw: rows per workgroup, up to PC_WAVES (the host's search_block).
 __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
     SegSearch seg, int64_t ldw, int R, int nc, int64_t ldu,
-    int metric) {
+    int metric, int rpw) {
   const float* __restrict__ W = seg.W[blockIdx.y];
   const float* __restrict__ U = seg.U[blockIdx.y];
   const SearchWs s = seg.s[blockIdx.y];
@@ -888,10 +890,10 @@ __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
   if (c1 < nc) { const float dg = U[(int64_t)c1 * ldu + c1]; d21 = dg * dg; }
   const int n = (int)wave_sum_f((in0 ? 1.f : 0.f) + (in1 ? 1.f : 0.f));
   SortedRow& sr = rows[wv];
-  for (int r0 = blockIdx.x * PC_WAVES; r0 < R; r0 += gridDim.x * PC_WAVES) {
+  for (int r0 = blockIdx.x * rpw; r0 < R; r0 += gridDim.x * rpw) {
     const int row = r0 + wv;
     __syncthreads();                       // previous rows' errs consumed
-    if (row < R) {
+    if (wv < rpw && row < R) {
       float x0 = in0 ? target_of(W[(int64_t)row * ldw + c0], d20, metric) : INFINITY;
       float x1 = in1 ? target_of(W[(int64_t)row * ldw + c1], d21, metric) : INFINITY;
       wave_sort128(x0, x1);
@@ -900,14 +902,14 @@ __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
     }
     __syncthreads();
     // the workgroup's (row, candidate) pairs spread over all its lanes
-    for (int pq = tid; pq < PC_WAVES * NQ; pq += 64 * PC_WAVES) {
+    for (int pq = tid; pq < rpw * NQ; pq += 64 * PC_WAVES) {
       const int q = pq / NQ, k = pq - q * NQ;
       if (r0 + q < R) {
         errs[q][k] = split_err(rows[q], n, pv[k]);
       }
     }
     __syncthreads();
-    const int nr = min(PC_WAVES, R - r0);
+    const int nr = min(rpw, R - r0);
     for (int k = tid; k < NQ; k += 64 * PC_WAVES) {
       double v = acc[k];
       for (int w = 0; w < nr; ++w) v += errs[w][k];
@@ -1371,20 +1373,40 @@ static int search_block(const SegSearch& seg, int nseg, int64_t ldw, int R, int 
                         int64_t ldu, int metric, int up_lim, hipStream_t st) {
   const int ncand = up_lim - 1;
   const int nwg_cs = (int)std::min<int64_t>(cdiv(R, CS_PH), CS_MAXWG);
-  const int nwg_q = (int)cdiv(R, Q_RPW);
-  const int nwg_c = (int)std::min<int64_t>(cdiv(R, PC_WAVES), PX_MAXWG);
-  // phase A: ceil(ncand / PR_CW) workgroups of up to PR_CW candidates per
-  // 64-row group (at least PR_MINW wavefronts: the reduction's 576 threads)
-  const int ncg = (int)cdiv(ncand, PR_CW), cw = (int)cdiv(ncand, ncg);
+  // Few rows leave most CUs idle, and a block is then its launches' latency:
+  // smaller workgroups, the same sums.  Whole loops with this (us per block, before
+  // / after): 256 rows 88 / 70, 768 88 / 73, 1000 88 / 76, 1536 93 / 83, 2048
+  // 96 / 89; 4096 110, unchanged.
+  // Quantile passes: Q_RPW_S rows per workgroup while that gives at most one
+  // workgroup per CU (at 3072 rows 103 against 100, at 4096 119 against 110; 4
+  // rows: 75 at 768 rows, 99 at 2048).
+  const bool qs = R <= 2048;
+  const int nwg_q = (int)cdiv(R, qs ? Q_RPW_S : Q_RPW);
+  // phase C: 8 rows per workgroup up to 2048 rows, whose 648 (row, candidate)
+  // pairs are one round over its 1024 lanes (16 rows: two) on twice as many
+  // CUs; above, 16 rows, as many workgroups as its partials hold
+  const int rpw = R <= 8 * PX_MAXWG ? PC_WAVES / 2 : PC_WAVES;
+  const int nwg_c = (int)std::min<int64_t>(cdiv(R, rpw), PX_MAXWG);
+  // phase A: ncg workgroups of up to PR_CW candidates per 64-row group (at
+  // least PR_MINW wavefronts: the reduction's 576 threads): as few as hold
+  // the candidates, or as many as fill 256 CUs where rows are few (a
+  // candidate's sums do not depend on it)
   const int nrg = (int)std::min<int64_t>(cdiv(R, 64), PX_MAXWG);
+  const int ncg0 = std::max((int)cdiv(ncand, PR_CW), std::min(ncand, PX_MAXWG / (nrg * nseg)));
+  const int cw = (int)cdiv(ncand, ncg0), ncg = (int)cdiv(ncand, cw);
   const unsigned y = (unsigned)nseg;
   k_colscore<<<dim3(nwg_cs, y), CS_THREADS, 0, st>>>(seg, ldw, R, nc, ldu, metric);
   k_phase_a_rows<<<dim3(nrg * ncg, y), 64 * std::max(cw, PR_MINW), 0, st>>>(
       seg, ldw, R, nc, ldu, metric, ncand, up_lim, ncg, cw);
-  k_qpass1<<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
-  k_qlist<<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
+  if (qs) {
+    k_qpass1<Q_RPW_S><<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
+    k_qlist<Q_RPW_S><<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
+  } else {
+    k_qpass1<Q_RPW><<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
+    k_qlist<Q_RPW><<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
+  }
   k_qselect<<<dim3(NT, y), QS_T, 0, st>>>(seg, R, nc);
-  k_phase_c<<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu, metric);
+  k_phase_c<<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu, metric, rpw);
   CRBQ_LAUNCH_CHECK();
   return CRBQ_OK;
 }

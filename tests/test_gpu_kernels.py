@@ -677,3 +677,11 @@ def test_block_search_candidate_layouts_vs_oracle(R, up_lim):
     assert np.max(np.abs(ea - eo) / np.abs(eo)) < 1e-4
     assert gt["i_star"] == tr.i_star
     np.testing.assert_array_equal((masks.cpu() == 3).numpy(), m3_o.numpy())
+
+
+@pytest.mark.parametrize("R", [7, 9, 65, 2047, 2049])
+def test_block_search_row_split_edges(R):
+    """Row counts at the edges of the search's workgroups (8 rows and the
+    candidates spread over many workgroups up to 2048 rows, 16 and 32 rows and
+    few workgroups above), against the oracle like the other layouts."""
+    test_block_search_candidate_layouts_vs_oracle(R, 50)
