@@ -161,6 +161,8 @@ def percentiles_cpu() -> torch.Tensor:
 def ready(device: torch.device | None = None) -> ctypes.CDLL:
     """Library handle, after checking the device is a gfx950 and uploading
     the percentile table (once per device)."""
+    if device is not None and device.index in _ready_devices:
+        return _lib
     lib = load()
     if not torch.cuda.is_available():
         raise CrbqError("no HIP device: the crbq path runs only on an MI355X (gfx950)")

@@ -313,7 +313,9 @@ def binarize(x: torch.Tensor, mask: torch.Tensor, order: int, method: str, lam: 
     except RuntimeError as e:
         raise _lib.CrbqError(f"binarize: mask of shape {tuple(mask.shape)} does not "
                              f"broadcast to {tuple(xf.shape)}") from e
-    m = m.to(torch.uint8).contiguous()
+    # a bool mask is the kernel's 0 / 1 bytes as it is
+    m = m.view(torch.uint8) if m.dtype == torch.bool else m.to(torch.uint8)
+    m = m.contiguous()
     R, nc = xf.shape
     if out is None:
         out = torch.empty((R, nc), dtype=torch.float32, device=x.device)

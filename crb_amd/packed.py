@@ -61,19 +61,17 @@ class PackedLinear(nn.Module):
         """The dense quantized weight (bit-identical to what was packed)."""
         return kernels.unpack(self.codes, self.lut, self.sal, self.in_features, self.ex)
 
-    def _fused(self, x: torch.Tensor) -> bool:
-        """Product, exceptions, bias and rounding in one kernel: activations
-        and bias in the weights' dtype and few exceptions."""
-        b = self.bias
-        return (x.dtype == self.lut.dtype and self.ex_idx.numel() <= LINEAR_MAX_EX
-                and (b is None or (b.dtype == x.dtype and b.is_contiguous())))
-
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
-        if x2.shape[0] <= GEMM_MAX_TOKENS and self._fused(x):
-            y = kernels.linear_packed(self.codes, self.lut, self.sal, self.in_features, x2,
-                                      self.bias, self.ex)
+        b = self._buffers            # one token's call is host time: no attribute look-ups
+        lut, bias, n_ex = b["lut"], b["bias"], b["ex_idx"].numel()
+        # product, exceptions, bias and rounding in one kernel: activations and
+        # bias in the weights' dtype and few exceptions
+        if (x2.shape[0] <= GEMM_MAX_TOKENS and x.dtype == lut.dtype and n_ex <= LINEAR_MAX_EX
+                and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()))):
+            y = kernels.linear_packed(b["codes"], lut, b["sal"], self.in_features, x2, bias,
+                                      self.ex if n_ex else None)
         elif x2.shape[0] <= GEMM_MAX_TOKENS:
             mm = kernels.gemv_packed if x2.shape[0] <= GEMV_MAX_TOKENS else kernels.gemm_packed
             y = mm(self.codes, self.lut, self.sal, self.in_features, x2, self.ex)
