@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void k_fallback_u(const float* __restrict__ H,
 
 // Diagonal block: Cholesky factor L and its inverse X = L^-1 of one
 // bj x bj block (bj <= NB; rows past bj are padded with the identity), in
-// place in LDS.  256 threads = 4 wavefronts.  The block is split
+// place in LDS.  512 threads = 8 wavefronts.  The block is split
 // recursively like the whole matrix (X11, T = A21 X11^T, A22 -= T T^T,
 // A21 = T X11, X22, X21 = -X22 A21):
 //  * 16 x 16 leaves: one wavefront, lane i & 15 holding row i in
@@ -188,14 +188,24 @@ __global__ __launch_bounds__(256) void k_fallback_u(const float* __restrict__ H,
 //  * 32 x 32 blocks: one wavefront runs both leaves and the four 16 x 16
 //    products (v_mfma_f32_16x16x4f32), so no workgroup barrier is needed.
 //  * the 64 and 128 levels: the products' 16 x 16 output tiles are spread
-//    over the 4 wavefronts, one barrier between dependent products.
+//    over the 8 wavefronts, one barrier between dependent products.
 // This factorization need not follow the reference's rounding step for
 // step (LAPACK's blocked potrf does not either), so it uses fused
 // multiply-adds and hardware square root and reciprocal per pivot.
-constexpr int LDP = NB + 1;            // LDS pitch of the block (column reads conflict-free)
+// What bounds it is the latency of its one-wavefront 32-row blocks (leaves
+// and dependent MFMA chains), then the products' MFMAs; two wavefronts per
+// SIMD hide the products' LDS reads, and a pitch of 140 floats puts the 16
+// rows x 4 columns of an operand read on 64 different banks and lets the
+// block be filled with 16-byte stores.  Interleaving each leaf's inverse
+// with its factorization hides the pivot's square root and reciprocal.
+// With 4 wavefronts, a pitch of 129 and the leaf's two passes one after the
+// other the factor took 2406 us at C = 4096, 1046 at 2048 and 376 at 768;
+// now 2329, 999 and 357, every bit of U the same.
+constexpr int NWV = 8;                 // wavefronts of a diagonal block or node
+constexpr int LDP = NB + 12;           // LDS pitch of the block: 16 rows x 4 columns on 64 banks
 constexpr int TSP = NB / 2 + 1;        // LDS pitch of the product scratch T
 
-struct DiagSmem {
+struct __attribute__((aligned(16))) DiagSmem {
   float Ls[NB][LDP];
   float Ts[(NB / 2) * TSP];
   int fail;
@@ -290,46 +300,52 @@ __device__ __forceinline__ float fnma_row_bcast(float d, float s, float m, int l
 __device__ __forceinline__ void leaf16(DiagSmem& sm, int o, int lane, int off, int bj,
                                        int* info) {
   const int i = lane & 15;
-  float a[16], rdg[16];
+  float a[16], y[16];
 #pragma unroll
   for (int c = 0; c < 16; ++c) a[c] = sm.Ls[o + i][o + c];
+#pragma unroll
+  for (int s = 0; s < 16; ++s) y[s] = i == s ? 1.f : 0.f;
   unsigned badm = 0u;   // bad pivots as bits (the same in every lane)
+  float piv = row_bcast(a[0], 0);
+  float rd = __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(piv));
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const float piv = row_bcast(a[j], j);
     badm |= (!(piv > 0.f) && o + j < bj) ? (1u << j) : 0u;
-    const float rd = __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(piv));
-    rdg[j] = rd;
     a[j] *= rd;
+    y[j] *= rd;
     // a[k] -= L[i][j] L[k][j]; the first update reads a[j] right after its
-    // scaling, and the next column's pivot reads a[j + 1] (written by the
-    // first update) at most two updates later
+    // scaling, and the next pivot's broadcast reads a[j + 1] right after that
+    // update.  The next pivot's square root and reciprocal are issued
+    // between the column's other updates, which hide them.
+    float sq = 0.f;
+    if (j < 15) {
+      a[j + 1] = fnma_row_bcast<true, true>(a[j + 1], a[j], a[j], j + 1);
+      piv = row_bcast(a[j + 1], j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int k = j + 2; k < 16; ++k) a[k] = fnma_row_bcast<false, false>(a[k], a[j], a[j], k);
+    if (j < 15) {
+      sq = __builtin_amdgcn_sqrtf(piv);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // X: every later row's accumulator takes its term once y[j] is known, so
+    // each receives k = 0, 1, ... in the order of a row-by-row dot product
 #pragma unroll
     for (int k = j + 1; k < 16; ++k) {
-      if (k == j + 1 && k == 15) a[k] = fnma_row_bcast<true, true>(a[k], a[j], a[j], k);
-      else if (k == j + 1) a[k] = fnma_row_bcast<true, false>(a[k], a[j], a[j], k);
-      else if (k == 15) a[k] = fnma_row_bcast<false, true>(a[k], a[j], a[j], k);
-      else a[k] = fnma_row_bcast<false, false>(a[k], a[j], a[j], k);
+      y[k] = fnma_row_bcast<false, false>(y[k], a[j], y[j], k);
+      if (k == (j + 16) / 2) {
+        rd = __builtin_amdgcn_rcpf(sq);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
+    if (j == 14) rd = __builtin_amdgcn_rcpf(sq);
   }
   const unsigned bm = __builtin_amdgcn_readfirstlane(badm);
   const int bad = bm ? __builtin_ctz(bm) : 16;   // first bad pivot
   if (bad < 16 && lane == 0) {
     sm.fail = 1;
     atomicCAS(info, 0, off + o + bad + 1);
-  }
-  // right-looking: once y[r] is known every later row's accumulator takes
-  // its term, so each accumulator receives k = 0, 1, ... in the same order
-  // as a row-by-row dot product would, while the dependent chain is one
-  // multiply and one fma per row
-  float y[16], acc[16];
-#pragma unroll
-  for (int s = 0; s < 16; ++s) acc[s] = i == s ? 1.f : 0.f;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    y[r] = acc[r] * rdg[r];
-#pragma unroll
-    for (int s = r + 1; s < 16; ++s) acc[s] = fnma_row_bcast<false, false>(acc[s], a[r], y[r], s);
   }
   if (lane < 16) {
 #pragma unroll
@@ -382,24 +398,26 @@ __device__ __forceinline__ void lower_tile(int e, int& ti, int& tj) {
 }
 
 // The products of a level with H-row halves at (o, o), 16 x 16 tiles over
-// the 4 wavefronts.  Full-depth products (the triangular operands' zero
-// halves included) so that every operand read of a tile can be issued
-// before its MFMA chain, with a wavefront's tiles interleaved.  Ends with a
-// barrier.
+// the wavefronts.  Full-depth products (the triangular operands' zero halves
+// included) so that every operand read of a tile can be issued before its
+// MFMA chain, with a wavefront's tiles interleaved (tiles past the last
+// repeat it and are not stored).  Ends with a barrier.
 template <int H>
 __device__ __forceinline__ void level_panel(DiagSmem& sm, int o, int wv, int lane) {
-  constexpr int NTL = H / 16, TPW = NTL * NTL / 4, NL = NTL * (NTL + 1) / 2;
-  constexpr int LPW = (NL + 3) / 4;
+  constexpr int NTL = H / 16, NF = NTL * NTL, NL = NTL * (NTL + 1) / 2;
+  constexpr int TPW = (NF + NWV - 1) / NWV, LPW = (NL + NWV - 1) / NWV;
   const int lr = lane & 15, lk = lane >> 4, p = o + H;
-  {                                            // T = A21 X11^T
-    f4_t t[TPW];
-    int ti[TPW], tj[TPW];
+  int ti[TPW], tj[TPW];
 #pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-      ti[q] = (wv + 4 * q) / NTL;
-      tj[q] = (wv + 4 * q) % NTL;
-      t[q] = f4_t{0.f, 0.f, 0.f, 0.f};
-    }
+  for (int q = 0; q < TPW; ++q) {
+    const int e = min(wv + NWV * q, NF - 1);
+    ti[q] = e / NTL;
+    tj[q] = e % NTL;
+  }
+  if (wv < NF) {                               // T = A21 X11^T
+    f4_t t[TPW];
+#pragma unroll
+    for (int q = 0; q < TPW; ++q) t[q] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < H; k += 4)
 #pragma unroll
@@ -408,54 +426,56 @@ __device__ __forceinline__ void level_panel(DiagSmem& sm, int o, int wv, int lan
                      sm.Ls[o + 16 * tj[q] + lr][o + k + lk], t[q]);
 #pragma unroll
     for (int q = 0; q < TPW; ++q)
+      if (wv + NWV * q < NF) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sm.Ts[(16 * ti[q] + 4 * lk + r) * TSP + 16 * tj[q] + lr] = t[q][r];
+        for (int r = 0; r < 4; ++r)
+          sm.Ts[(16 * ti[q] + 4 * lk + r) * TSP + 16 * tj[q] + lr] = t[q][r];
+      }
   }
   __syncthreads();
-  {                                            // A22 -= T T^T (lower tiles)
+  if (wv < NL) {                               // A22 -= T T^T (lower tiles)
     f4_t s[LPW];
-    int ti[LPW], tj[LPW];
+    int si[LPW], sj[LPW];
 #pragma unroll
     for (int q = 0; q < LPW; ++q) {
-      const int e = wv + 4 * q;
-      lower_tile(e < NL ? e : NL - 1, ti[q], tj[q]);
+      const int e = wv + NWV * q;
+      lower_tile(e < NL ? e : NL - 1, si[q], sj[q]);
       s[q] = f4_t{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int k = 0; k < H; k += 4)
 #pragma unroll
       for (int q = 0; q < LPW; ++q)
-        s[q] = mfma4(sm.Ts[(16 * ti[q] + lr) * TSP + k + lk],
-                     sm.Ts[(16 * tj[q] + lr) * TSP + k + lk], s[q]);
-    f4_t u[TPW];                               // A21 = T X11
-    int ui[TPW], uj[TPW];
-#pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-      ui[q] = (wv + 4 * q) / NTL;
-      uj[q] = (wv + 4 * q) % NTL;
-      u[q] = f4_t{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int k = 0; k < H; k += 4)
-#pragma unroll
-      for (int q = 0; q < TPW; ++q)
-        u[q] = mfma4(sm.Ts[(16 * ui[q] + lr) * TSP + k + lk],
-                     sm.Ls[o + k + lk][o + 16 * uj[q] + lr], u[q]);
+        s[q] = mfma4(sm.Ts[(16 * si[q] + lr) * TSP + k + lk],
+                     sm.Ts[(16 * sj[q] + lr) * TSP + k + lk], s[q]);
 #pragma unroll
     for (int q = 0; q < LPW; ++q) {
-      if (wv + 4 * q < NL) {
+      if (wv + NWV * q < NL) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int rr = 16 * ti[q] + 4 * lk + r, cc = 16 * tj[q] + lr;
+          const int rr = 16 * si[q] + 4 * lk + r, cc = 16 * sj[q] + lr;
           if (cc <= rr) sm.Ls[p + rr][p + cc] -= s[q][r];
         }
       }
     }
+  }
+  if (wv < NF) {                               // A21 = T X11
+    f4_t u[TPW];
+#pragma unroll
+    for (int q = 0; q < TPW; ++q) u[q] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < H; k += 4)
+#pragma unroll
+      for (int q = 0; q < TPW; ++q)
+        u[q] = mfma4(sm.Ts[(16 * ti[q] + lr) * TSP + k + lk],
+                     sm.Ls[o + k + lk][o + 16 * tj[q] + lr], u[q]);
 #pragma unroll
     for (int q = 0; q < TPW; ++q)
+      if (wv + NWV * q < NF) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sm.Ls[p + 16 * ui[q] + 4 * lk + r][o + 16 * uj[q] + lr] = u[q][r];
+        for (int r = 0; r < 4; ++r)
+          sm.Ls[p + 16 * ti[q] + 4 * lk + r][o + 16 * tj[q] + lr] = u[q][r];
+      }
   }
   __syncthreads();
 }
@@ -464,27 +484,33 @@ __device__ __forceinline__ void level_panel(DiagSmem& sm, int o, int wv, int lan
 // registers until every wavefront has read A21.  Ends with a barrier.
 template <int H>
 __device__ __forceinline__ void level_x21(DiagSmem& sm, int o, int wv, int lane) {
-  constexpr int NTL = H / 16, TPW = NTL * NTL / 4;
+  constexpr int NTL = H / 16, NF = NTL * NTL, TPW = (NF + NWV - 1) / NWV;
   const int lr = lane & 15, lk = lane >> 4, p = o + H;
   f4_t x[TPW];
   int ti[TPW], tj[TPW];
 #pragma unroll
   for (int q = 0; q < TPW; ++q) {
-    ti[q] = (wv + 4 * q) / NTL;
-    tj[q] = (wv + 4 * q) % NTL;
+    const int e = min(wv + NWV * q, NF - 1);
+    ti[q] = e / NTL;
+    tj[q] = e % NTL;
     x[q] = f4_t{0.f, 0.f, 0.f, 0.f};
   }
+  if (wv < NF) {
 #pragma unroll
-  for (int k = 0; k < H; k += 4)
+    for (int k = 0; k < H; k += 4)
 #pragma unroll
-    for (int q = 0; q < TPW; ++q)
-      x[q] = mfma4(sm.Ls[p + 16 * ti[q] + lr][p + k + lk], sm.Ls[p + k + lk][o + 16 * tj[q] + lr],
-                   x[q]);
+      for (int q = 0; q < TPW; ++q)
+        x[q] = mfma4(sm.Ls[p + 16 * ti[q] + lr][p + k + lk], sm.Ls[p + k + lk][o + 16 * tj[q] + lr],
+                     x[q]);
+  }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < TPW; ++q)
+    if (wv + NWV * q < NF) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sm.Ls[p + 16 * ti[q] + 4 * lk + r][o + 16 * tj[q] + lr] = -x[q][r];
+      for (int r = 0; r < 4; ++r)
+        sm.Ls[p + 16 * ti[q] + 4 * lk + r][o + 16 * tj[q] + lr] = -x[q][r];
+    }
   __syncthreads();
 }
 
@@ -503,15 +529,15 @@ __device__ __forceinline__ bool block64(DiagSmem& sm, int o, int wv, int lane, i
 }
 
 // Load the bj x bj diagonal block at (off, off) into sm.Ls: lower triangle,
-// identity padding, zero above; 16 coalesced 4-float groups per thread,
-// all in flight together.  Ends with a barrier.
-__device__ __forceinline__ void diag_load(DiagSmem& sm, const float* A, int64_t lda, int off,
-                                          int bj, bool vec) {
+// identity padding, zero above; 4-float groups, each thread's all in flight
+// together (block_fetch, then block_put; a barrier is the caller's).
+constexpr int NG = NB * NB / 4 / (64 * NWV);     // groups per thread
+__device__ __forceinline__ void block_fetch(float (&v)[NG][4], const float* A, int64_t lda,
+                                            int off, int bj, bool vec) {
   const int tid = threadIdx.x;
-  float v[16][4];
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
-    const int f = tid + 256 * u, i = f >> 5, j0 = (f & 31) * 4;
+  for (int u = 0; u < NG; ++u) {
+    const int f = tid + 64 * NWV * u, i = f >> 5, j0 = (f & 31) * 4;
     const float* src = A + (int64_t)(off + i) * lda + off + j0;
     if (vec && i < bj && j0 + 3 < bj) {
       const float4 q = *(const float4*)src;
@@ -521,17 +547,21 @@ __device__ __forceinline__ void diag_load(DiagSmem& sm, const float* A, int64_t 
       for (int c = 0; c < 4; ++c) v[u][c] = (i < bj && j0 + c < bj) ? src[c] : 0.f;
     }
   }
+}
+__device__ __forceinline__ void block_put(DiagSmem& sm, const float (&v)[NG][4], int bj) {
+  const int tid = threadIdx.x;
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
-    const int f = tid + 256 * u, i = f >> 5, j0 = (f & 31) * 4;
+  for (int u = 0; u < NG; ++u) {
+    const int f = tid + 64 * NWV * u, i = f >> 5, j0 = (f & 31) * 4;
+    f4_t q;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const int j = j0 + c;
-      sm.Ls[i][j] = (i < bj && j <= i) ? v[u][c] : (i == j ? 1.f : 0.f);
+      q[c] = (i < bj && j <= i) ? v[u][c] : (i == j ? 1.f : 0.f);
     }
+    *(f4_t*)&sm.Ls[i][j0] = q;
   }
   if (tid == 0) sm.fail = 0;
-  __syncthreads();
 }
 
 // X = L^-1 of the block in sm.Ls (L is not kept).  Returns false after a
@@ -551,8 +581,8 @@ __device__ __forceinline__ void diag_store(const DiagSmem& sm, float* A, int64_t
                                            int bj, bool vec) {
   const int tid = threadIdx.x;
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
-    const int f = tid + 256 * u, i = f >> 5, j0 = (f & 31) * 4;
+  for (int u = 0; u < NG; ++u) {
+    const int f = tid + 64 * NWV * u, i = f >> 5, j0 = (f & 31) * 4;
     float* dst = A + (int64_t)(off + i) * lda + off + j0;
     float q[4];
 #pragma unroll
@@ -571,14 +601,17 @@ __device__ __forceinline__ bool diag_vec(const float* A, int64_t lda, int off) {
   return ((lda & 3) == 0) && ((((uintptr_t)A) & 15) == 0) && ((off & 3) == 0);
 }
 
-__global__ __launch_bounds__(256) void k_chol_inv_diag(float* A, int64_t lda, int off, int bj,
-                                                       int* info) {
+__global__ __launch_bounds__(64 * NWV) void k_chol_inv_diag(float* A, int64_t lda, int off,
+                                                            int bj, int* info) {
   if (*info) return;
   __shared__ DiagSmem sm;
   // the wavefront index as a scalar, so branches on it are uniform
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool vec = diag_vec(A, lda, off);
-  diag_load(sm, A, lda, off, bj, vec);
+  float v[NG][4];
+  block_fetch(v, A, lda, off, bj, vec);
+  block_put(sm, v, bj);
+  __syncthreads();
   if (!diag_core(sm, w, lane, off, bj, info)) return;
   diag_store(sm, A, lda, off, bj, vec);
 }
@@ -598,16 +631,17 @@ __global__ __launch_bounds__(256) void k_chol_inv_diag(float* A, int64_t lda, in
 // and the same epilogues (T = acc, Q = acc, A22 = A22 - acc, X21 = -acc), so
 // X is bitwise what those launches give; the zero parts of the triangular
 // operands are skipped (exact zeros leave the sums unchanged).  Tiles go
-// to the 4 wavefronts in pairs of a short and a long K range (tile
-// columns or rows w and 7 - w), so every wavefront issues the same number
-// of MFMAs.
+// to the 8 wavefronts in pairs of a short and a long K range (tile
+// columns or rows w % 4 and 7 - w % 4, half of the other dimension each), so
+// every wavefront issues the same number of MFMAs.  A21 is loaded with A11
+// and A22 during the products before it is needed.
 struct NodeSmem {
   DiagSmem d;                // the diagonal block (X11, then A22 / X22)
   float P[NB][LDP];          // A21, then T, then Q
 };
 
-__global__ __launch_bounds__(256) void k_chol_inv_node(float* A, int64_t lda, int off, int n,
-                                                       int* info) {
+__global__ __launch_bounds__(64 * NWV) void k_chol_inv_node(float* A, int64_t lda, int off,
+                                                            int n, int* info) {
   if (*info) return;
   __shared__ NodeSmem nm;
   DiagSmem& sm = nm.d;
@@ -616,141 +650,151 @@ __global__ __launch_bounds__(256) void k_chol_inv_node(float* A, int64_t lda, in
   const int lr = lane & 15, lk = lane >> 4;
   const int n2 = n - NB;                          // 1 .. 128
   const bool vec = diag_vec(A, lda, off);
-  // ---- X11
-  diag_load(sm, A, lda, off, NB, vec);
-  if (!diag_core(sm, w, lane, off, NB, info)) return;
-  diag_store(sm, A, lda, off, NB, vec);
-  // ---- A21 (n2 x 128) into P, zero rows past n2
   float* A21 = A + (int64_t)(off + NB) * lda + off;
+  // ---- X11; A21 (n2 x 128) into P, zero rows past n2
   {
-    float v[16][4];
+    float v[NG][4], a[NG][4];
+    block_fetch(v, A, lda, off, NB, vec);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int f = tid + 256 * u, i = f >> 5, j0 = (f & 31) * 4;
+    for (int u = 0; u < NG; ++u) {
+      const int f = tid + 64 * NWV * u, i = f >> 5, j0 = (f & 31) * 4;
       const float* src = A21 + (int64_t)i * lda + j0;
       if (vec && i < n2) {
         const float4 q = *(const float4*)src;
-        v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
+        a[u][0] = q.x; a[u][1] = q.y; a[u][2] = q.z; a[u][3] = q.w;
       } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) v[u][c] = i < n2 ? src[c] : 0.f;
+        for (int c = 0; c < 4; ++c) a[u][c] = i < n2 ? src[c] : 0.f;
       }
     }
+    block_put(sm, v, NB);
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const int f = tid + 256 * u, i = f >> 5, j0 = (f & 31) * 4;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) P[i][j0 + c] = v[u][c];
+    for (int u = 0; u < NG; ++u) {
+      const int f = tid + 64 * NWV * u, i = f >> 5, j0 = (f & 31) * 4;
+      *(f4_t*)&P[i][j0] = f4_t{a[u][0], a[u][1], a[u][2], a[u][3]};
     }
   }
   __syncthreads();
-  // wavefront w's tile columns (T, Q) or rows (X21): w and 7 - w, 8 tiles each
-  const int ca = w, cb = 7 - w;
+  if (!diag_core(sm, w, lane, off, NB, info)) return;
+  float a22[NG][4];                               // in flight until the Schur tiles are done
+  block_fetch(a22, A, lda, off + NB, n2, vec);
+  diag_store(sm, A, lda, off, NB, vec);
+  // wavefront w's tile columns (T, Q) or rows (X21) and its half of the other
+  // dimension's tiles
+  const int ca = w & 3, cb = 7 - ca, h0 = (w >> 2) * 4;
   // ---- T = A21 X11^T: column tile j sums k < 16 (j + 1)
   {
-    f4_t ta[8], tb[8];
+    f4_t ta[4], tb[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { ta[i] = f4_t{0.f, 0.f, 0.f, 0.f}; tb[i] = ta[i]; }
+    for (int i = 0; i < 4; ++i) { ta[i] = f4_t{0.f, 0.f, 0.f, 0.f}; tb[i] = ta[i]; }
     const int ka = 16 * (ca + 1), kb = 16 * (cb + 1);   // ka < kb
+#pragma unroll 4
     for (int k = 0; k < kb; k += 4) {
       const float ba = sm.Ls[16 * ca + lr][k + lk], bb = sm.Ls[16 * cb + lr][k + lk];
-      float a[8];
+      float a[4];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) a[i] = P[16 * i + lr][k + lk];
+      for (int i = 0; i < 4; ++i) a[i] = P[16 * (h0 + i) + lr][k + lk];
       if (k < ka) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) ta[i] = mfma4(a[i], ba, ta[i]);
+        for (int i = 0; i < 4; ++i) ta[i] = mfma4(a[i], ba, ta[i]);
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) tb[i] = mfma4(a[i], bb, tb[i]);
+      for (int i = 0; i < 4; ++i) tb[i] = mfma4(a[i], bb, tb[i]);
     }
     __syncthreads();                              // every read of A21 done
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        P[16 * i + 4 * lk + r][16 * ca + lr] = ta[i][r];
-        P[16 * i + 4 * lk + r][16 * cb + lr] = tb[i][r];
+        P[16 * (h0 + i) + 4 * lk + r][16 * ca + lr] = ta[i][r];
+        P[16 * (h0 + i) + 4 * lk + r][16 * cb + lr] = tb[i][r];
       }
   }
   __syncthreads();
   // ---- S = T T^T (the 36 lower tiles, full K) and Q = T X11 (column tile j
   // sums k >= 16 j)
-  f4_t sacc[9];
-  int si[9], sj[9];
+  constexpr int SPW = (36 + NWV - 1) / NWV;
+  f4_t sacc[SPW];
+  int si[SPW], sj[SPW];
 #pragma unroll
-  for (int q = 0; q < 9; ++q) {
-    lower_tile(w + 4 * q, si[q], sj[q]);
+  for (int q = 0; q < SPW; ++q) {
+    lower_tile(min(w + NWV * q, 35), si[q], sj[q]);
     sacc[q] = f4_t{0.f, 0.f, 0.f, 0.f};
   }
+#pragma unroll 4
   for (int k = 0; k < NB; k += 4) {
 #pragma unroll
-    for (int q = 0; q < 9; ++q)
-      sacc[q] = mfma4(P[16 * si[q] + lr][k + lk], P[16 * sj[q] + lr][k + lk], sacc[q]);
+    for (int q = 0; q < SPW; ++q)
+      if (w + NWV * q < 36)
+        sacc[q] = mfma4(P[16 * si[q] + lr][k + lk], P[16 * sj[q] + lr][k + lk], sacc[q]);
   }
-  f4_t ua[8], ub[8];
+  f4_t ua[4], ub[4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) { ua[i] = f4_t{0.f, 0.f, 0.f, 0.f}; ub[i] = ua[i]; }
+  for (int i = 0; i < 4; ++i) { ua[i] = f4_t{0.f, 0.f, 0.f, 0.f}; ub[i] = ua[i]; }
   {
     const int ka = 16 * ca, kb = 16 * cb;         // start of the K range; ka < kb
+#pragma unroll 4
     for (int k = ka; k < NB; k += 4) {
       const float ba = sm.Ls[k + lk][16 * ca + lr], bb = sm.Ls[k + lk][16 * cb + lr];
-      float a[8];
+      float a[4];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) a[i] = P[16 * i + lr][k + lk];
+      for (int i = 0; i < 4; ++i) a[i] = P[16 * (h0 + i) + lr][k + lk];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) ua[i] = mfma4(a[i], ba, ua[i]);
+      for (int i = 0; i < 4; ++i) ua[i] = mfma4(a[i], ba, ua[i]);
       if (k >= kb) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) ub[i] = mfma4(a[i], bb, ub[i]);
+        for (int i = 0; i < 4; ++i) ub[i] = mfma4(a[i], bb, ub[i]);
       }
     }
   }
   __syncthreads();                                // every read of T and X11 done
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      P[16 * i + 4 * lk + r][16 * ca + lr] = ua[i][r];
-      P[16 * i + 4 * lk + r][16 * cb + lr] = ub[i][r];
+      P[16 * (h0 + i) + 4 * lk + r][16 * ca + lr] = ua[i][r];
+      P[16 * (h0 + i) + 4 * lk + r][16 * cb + lr] = ub[i][r];
     }
   // ---- A22 - S into the block buffer (rows and columns past n2: identity
   // padding, where S is 0), then X22
-  diag_load(sm, A, lda, off + NB, n2, vec);       // ends with a barrier
+  block_put(sm, a22, n2);
+  __syncthreads();
 #pragma unroll
-  for (int q = 0; q < 9; ++q)
+  for (int q = 0; q < SPW; ++q)
+    if (w + NWV * q < 36) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int rr = 16 * si[q] + 4 * lk + r, cc = 16 * sj[q] + lr;
-      if (cc <= rr) sm.Ls[rr][cc] = sm.Ls[rr][cc] - sacc[q][r];
+      for (int r = 0; r < 4; ++r) {
+        const int rr = 16 * si[q] + 4 * lk + r, cc = 16 * sj[q] + lr;
+        if (cc <= rr) sm.Ls[rr][cc] = sm.Ls[rr][cc] - sacc[q][r];
+      }
     }
   __syncthreads();
   if (!diag_core(sm, w, lane, off + NB, n2, info)) return;
   diag_store(sm, A, lda, off + NB, n2, vec);
   // ---- X21 = -X22 Q: row tile i sums k < 16 (i + 1)
   {
-    f4_t xa[8], xb[8];
+    f4_t xa[4], xb[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { xa[j] = f4_t{0.f, 0.f, 0.f, 0.f}; xb[j] = xa[j]; }
-    const int ra = ca, rb = cb;
-    const int ka = 16 * (ra + 1), kb = 16 * (rb + 1);
+    for (int j = 0; j < 4; ++j) { xa[j] = f4_t{0.f, 0.f, 0.f, 0.f}; xb[j] = xa[j]; }
+    const int ka = 16 * (ca + 1), kb = 16 * (cb + 1);
+#pragma unroll 4
     for (int k = 0; k < kb; k += 4) {
-      const float aa = sm.Ls[16 * ra + lr][k + lk], ab = sm.Ls[16 * rb + lr][k + lk];
-      float b[8];
+      const float aa = sm.Ls[16 * ca + lr][k + lk], ab = sm.Ls[16 * cb + lr][k + lk];
+      float b[4];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) b[j] = P[k + lk][16 * j + lr];
+      for (int j = 0; j < 4; ++j) b[j] = P[k + lk][16 * (h0 + j) + lr];
       if (k < ka) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xa[j] = mfma4(aa, b[j], xa[j]);
+        for (int j = 0; j < 4; ++j) xa[j] = mfma4(aa, b[j], xa[j]);
       }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) xb[j] = mfma4(ab, b[j], xb[j]);
+      for (int j = 0; j < 4; ++j) xb[j] = mfma4(ab, b[j], xb[j]);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int ia = 16 * ra + 4 * lk + r, ib = 16 * rb + 4 * lk + r, c = 16 * j + lr;
+        const int ia = 16 * ca + 4 * lk + r, ib = 16 * cb + 4 * lk + r, c = 16 * (h0 + j) + lr;
         if (ia < n2) A21[(int64_t)ia * lda + c] = -xa[j][r];
         if (ib < n2) A21[(int64_t)ib * lda + c] = -xb[j][r];
       }
@@ -799,12 +843,12 @@ static void carve_hinv(WsCarver& c, int64_t C, HinvWs& w) {
 static int chol_inv_rec(float* A, int64_t lda, int o, int n, HinvWs& w, float* Q,
                         hipStream_t s) {
   if (n <= NB) {
-    k_chol_inv_diag<<<1, 256, 0, s>>>(A, lda, o, n, w.info);
+    k_chol_inv_diag<<<1, 64 * NWV, 0, s>>>(A, lda, o, n, w.info);
     CRBQ_LAUNCH_CHECK();
     return CRBQ_OK;
   }
   if (n <= 2 * NB) {                  // split at NB: the whole node in one workgroup
-    k_chol_inv_node<<<1, 256, 0, s>>>(A, lda, o, n, w.info);
+    k_chol_inv_node<<<1, 64 * NWV, 0, s>>>(A, lda, o, n, w.info);
     CRBQ_LAUNCH_CHECK();
     return CRBQ_OK;
   }

@@ -485,6 +485,26 @@ def test_hinv_upper_ragged_levels(C):
     assert float((Ud.t() @ Ud @ Hdamp - torch.eye(C, dtype=torch.float64)).abs().max()) < 1e-3
 
 
+@pytest.mark.parametrize("C", [16, 113, 129, 145, 192, 255, 256, 257])
+def test_hinv_upper_node_edges(C):
+    """Edges of the one-workgroup block and node, whose tiles are spread over
+    8 wavefronts: a second half of 1, 17, 64, 127 and 128 rows, vector and
+    scalar row access (C a multiple of 4 or not), one row past a node.  To
+    first order the factor's relative error is at most C 2^-24 cond(H); the
+    bar is the smaller of that and the larger sizes' 1e-4."""
+    print(f"hinv node C={C}", flush=True)
+    H = _spd(C, C + 11).float()
+    U, retries, fb = _k().hinv_upper(H.to(DEV), None, 0.01)
+    torch.cuda.synchronize()
+    assert retries == 0 and not fb
+    Hdamp = H.double() + 0.01 * torch.diag(H.double()).mean() * torch.eye(C, dtype=torch.float64)
+    Uref = torch.linalg.cholesky(torch.linalg.inv(Hdamp), upper=True)
+    Uc = U.cpu()
+    assert torch.equal(torch.tril(Uc, -1), torch.zeros(C, C))
+    bar = min(1e-4, C * 2.0 ** -24 * float(torch.linalg.cond(Hdamp)))
+    assert rel(Uc, Uref.float()) < bar
+
+
 @pytest.mark.parametrize("C", [8192, 8320])
 def test_hinv_upper_large_vs_fp64(C):
     """Factors whose top-level products have >= 512 tiles of 128 x 128, so
