@@ -514,7 +514,7 @@ def linear_packed(codes: torch.Tensor, lut: torch.Tensor, sal: torch.Tensor, C: 
     x = _packed_x(x, lut, C, "linear_packed")
     T, R = x.shape[0], codes.shape[0]
     if bias is not None and (bias.dtype != lut.dtype or tuple(bias.shape) != (R,)
-                             or bias.stride(0) != 1):
+                             or not bias.is_contiguous()):
         raise _lib.CrbqError("linear_packed takes a contiguous [R] bias in the weights' dtype")
     y = torch.empty((T, R), dtype=lut.dtype, device=x.device)
     lib = _lib.ready(x.device)

@@ -67,9 +67,12 @@ class PackedLinear(nn.Module):
         b = self._buffers            # one token's call is host time: no attribute look-ups
         lut, bias, n_ex = b["lut"], b["bias"], b["ex_idx"].numel()
         # product, exceptions, bias and rounding in one kernel: activations and
-        # bias in the weights' dtype and few exceptions
+        # bias in the weights' dtype, few exceptions, a plain [R] bias (one that
+        # broadcasts or takes a gradient is added on its own)
         if (x2.shape[0] <= GEMM_MAX_TOKENS and x.dtype == lut.dtype and n_ex <= LINEAR_MAX_EX
-                and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()))):
+                and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()
+                                      and bias.shape == (self.out_features,)
+                                      and not bias.requires_grad))):
             y = kernels.linear_packed(b["codes"], lut, b["sal"], self.in_features, x2, bias,
                                       self.ex if n_ex else None)
         elif x2.shape[0] <= GEMM_MAX_TOKENS:

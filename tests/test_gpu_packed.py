@@ -270,3 +270,21 @@ def test_linear_packed_against_float64(R, C, T, dtype, bias, n_odd):
     err = (y.double().cpu() - ref).abs()
     assert (err <= half_ulp * ref.abs() + 1.1e-5 * scale + 2.0 ** -25).all()
     assert torch.equal(PackedLinear(codes, lut, sal, C, b, ex)(x), y)
+
+
+def test_packed_linear_bias_forms():
+    """A bias that broadcasts or takes a gradient is added on its own, as
+    before the product kernels took the bias."""
+    from crb_amd.packed import PackedLinear
+    q, masks = structured(48, 256, seed=5)
+    Q = _q16(q, torch.float16)
+    codes, lut, sal, ex = _k().pack(Q, torch.from_numpy(masks).to(DEV))
+    x = torch.randn(20, 256, generator=torch.Generator().manual_seed(1)).half().to(DEV)
+    plain = PackedLinear(codes, lut, sal, 256, None, ex)(x)
+    one = torch.full((1,), 0.5, dtype=torch.float16, device=DEV)
+    assert torch.equal(PackedLinear(codes, lut, sal, 256, one, ex)(x), plain + one)
+    b = torch.linspace(-1, 1, 48, device=DEV).half().requires_grad_()
+    y = PackedLinear(codes, lut, sal, 256, b, ex)(x)
+    assert torch.equal(y, plain + b)
+    y.sum().backward()
+    assert torch.equal(b.grad, torch.full_like(b, 20.0))
