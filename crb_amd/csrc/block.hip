@@ -862,10 +862,11 @@ __device__ __forceinline__ void wave_prefix(SortedRow& r, float x0, float x1, in
 // fp64 prefix sums of v and v^2; then the workgroup's (row, candidate k)
 // pairs over all its lanes, each two binary searches per group and range
 // sums (group_err1); the last workgroup takes k* = first strict minimum.
-// rpw: rows per workgroup, up to PC_WAVES (the host's search_block).
+// RPW: rows per workgroup, up to PC_WAVES (the host's search_block).
+template <int RPW>
 __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
     SegSearch seg, int64_t ldw, int R, int nc, int64_t ldu,
-    int metric, int rpw) {
+    int metric) {
   const float* __restrict__ W = seg.W[blockIdx.y];
   const float* __restrict__ U = seg.U[blockIdx.y];
   const SearchWs s = seg.s[blockIdx.y];
@@ -890,10 +891,10 @@ __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
   if (c1 < nc) { const float dg = U[(int64_t)c1 * ldu + c1]; d21 = dg * dg; }
   const int n = (int)wave_sum_f((in0 ? 1.f : 0.f) + (in1 ? 1.f : 0.f));
   SortedRow& sr = rows[wv];
-  for (int r0 = blockIdx.x * rpw; r0 < R; r0 += gridDim.x * rpw) {
+  for (int r0 = blockIdx.x * RPW; r0 < R; r0 += gridDim.x * RPW) {
     const int row = r0 + wv;
     __syncthreads();                       // previous rows' errs consumed
-    if (wv < rpw && row < R) {
+    if (wv < RPW && row < R) {
       float x0 = in0 ? target_of(W[(int64_t)row * ldw + c0], d20, metric) : INFINITY;
       float x1 = in1 ? target_of(W[(int64_t)row * ldw + c1], d21, metric) : INFINITY;
       wave_sort128(x0, x1);
@@ -902,14 +903,14 @@ __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
     }
     __syncthreads();
     // the workgroup's (row, candidate) pairs spread over all its lanes
-    for (int pq = tid; pq < rpw * NQ; pq += 64 * PC_WAVES) {
+    for (int pq = tid; pq < RPW * NQ; pq += 64 * PC_WAVES) {
       const int q = pq / NQ, k = pq - q * NQ;
       if (r0 + q < R) {
         errs[q][k] = split_err(rows[q], n, pv[k]);
       }
     }
     __syncthreads();
-    const int nr = min(rpw, R - r0);
+    const int nr = min(RPW, R - r0);
     for (int k = tid; k < NQ; k += 64 * PC_WAVES) {
       double v = acc[k];
       for (int w = 0; w < nr; ++w) v += errs[w][k];
@@ -1406,7 +1407,11 @@ static int search_block(const SegSearch& seg, int nseg, int64_t ldw, int R, int 
     k_qlist<Q_RPW><<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
   }
   k_qselect<<<dim3(NT, y), QS_T, 0, st>>>(seg, R, nc);
-  k_phase_c<<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu, metric, rpw);
+  if (rpw == PC_WAVES)
+    k_phase_c<PC_WAVES><<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu, metric);
+  else
+    k_phase_c<PC_WAVES / 2><<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu,
+                                                                      metric);
   CRBQ_LAUNCH_CHECK();
   return CRBQ_OK;
 }
