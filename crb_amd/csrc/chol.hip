@@ -294,9 +294,9 @@ __device__ __forceinline__ float fnma_row_bcast(float d, float s, float m, int l
 //  * Cholesky with lane i holding row i: at column j the pivot comes from
 //    lane j and L[k][j] from lane k (row broadcasts); lanes i <= j keep
 //    scratch in column j, never read.
-//  * Inverse with lane c holding column c of X: forward substitution
-//    X[r][c] = (delta_rc - sum_{k<r} L[r][k] X[k][c]) / L[r][r], the L
-//    values broadcast from lane r, so no lane masks are needed.
+//  * Inverse with lane c holding column c of X, in the same pass: once
+//    y[j] = X[j][c] is known every later row takes its term L[k][j] X[j][c]
+//    (L[k][j] from lane k), so no lane masks are needed.
 __device__ __forceinline__ void leaf16(DiagSmem& sm, int o, int lane, int off, int bj,
                                        int* info) {
   const int i = lane & 15;

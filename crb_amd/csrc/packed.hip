@@ -859,11 +859,10 @@ __global__ __launch_bounds__(256) void k_gemm_packed_sum(const float* __restrict
 // number of column splits (of at least 2 blocks) with the least modelled
 // time: rounds of one workgroup per CU, each 5 us and 0.7 + 2.1 tt / 128 us a
 // block, and a sum launch of 3.5 us and the partials written and read at 4
-// TB/s.  Measured against
-// splits to fill the chip once, twice (us): 4096 x 16384 at 300 tokens 74 /
-// 83, at 768 167 / 151, 4096 x 4096 at 300 33 / 34, at 768 57 / 65; against no
-// split, 4096 x 1920 at 64 16 / 26, 1024 x 1024 at 128 18.5 / 24.  One-tile
-// products of up to 8 blocks take no workspace.
+// TB/s.  Measured against splits to fill the chip once, twice (us): 4096 x
+// 16384 at 300 tokens 74 / 83, at 768 167 / 151, 4096 x 4096 at 300 33 / 34, at
+// 768 57 / 65; against no split, 4096 x 1920 at 64 16 / 26, 1024 x 1024 at 128
+// 18.5 / 24.  One-tile products of up to 8 blocks take no workspace.
 struct GmPlan {
   int tg, tt, ns, bps;
   int64_t row_tiles, tok_tiles;
