@@ -7,9 +7,13 @@ row, one salient-column bitmap per block; the format is described in
 include/crbq.h) and multiplies with them directly: up to 16 tokens per call
 through the packed GEMV (MFMA on weights decoded in registers), up to 768
 through the packed GEMM (each decoded fragment reused for up to 128 tokens),
-with bias and rounding in the same kernels, and larger batches, where the product is compute-bound, by unpacking into a
-temporary dense weight for the dense GEMM.  The limits are the measured
-crossovers on MI355X (4096 x 16384 and 16384 x 4096 fp16 layers).
+with bias and rounding in the same kernels, and larger batches, where the
+product is compute-bound, by unpacking into a temporary dense weight for the
+dense GEMM.  Packed / through the dense weight on MI355X, us: 4096 x 16384 at
+256 / 512 / 768 / 1024 tokens 63 / 99, 104 / 120, 158 / 138, 183 / 165; 16384 x
+4096 60 / 71, 94 / 90, 168 / 110, 185 / 130; 4096 x 4096 29 / 37, 40 / 40, 56 /
+43, 60 / 50; 1024 x 4096 21 / 37, 24 / 36, 26 / 36, 29 / 36.  Up to 768 tokens
+no temporary weight is allocated.
 """
 from __future__ import annotations
 
