@@ -477,25 +477,33 @@ __device__ __forceinline__ void for_ex(const PkEnd& e, int r_lo, int r_hi, int R
 // table) and the same columns of vector l & 15 (64 bytes), and feeds them to
 // four MFMAs as 8-column slices: the MFMA sums over k in any order as long
 // as A and B agree, so the columns need not be in the instruction's natural
-// k order.  The salient selectors are the same for every row: the workgroup
-// builds them once, in LDS, GV_SB blocks at a time.  The wavefronts' 16 x 16
+// k order.  The salient selectors are the same for every row: each
+// wavefront builds those of two blocks at a time, one per lane, in LDS of its
+// own, while the two blocks' loads are in flight (built for the whole
+// workgroup behind a barrier before the first load, us at 1 / 8 / 16 vectors:
+// 4096 x 16384 16.6 / 21.4 / 25.9, 16384 x 4096 17.0 / 21.7 / 27.6, 768 x 3072
+// 4.7 / 5.7 / 6.6, 4100 x 36000 45 / 58 / 76; now 15.3 / 20.0 / 25.1, 16.2 / 20.9 /
+// 26.2, 4.6 / 5.4 / 6.5, 41 / 52 / 72).  Bound by latency: four wavefronts per
+// SIMD, codes and tables in pieces of lines.  The wavefronts' 16 x 16
 // partial products are summed in LDS.  END: the result is rounded to the
 // weights' dtype after bias and exceptions, else fp32.
 constexpr int GV_WAVES = 16;
-constexpr int GV_SB = 256;        // blocks of selectors in LDS (32 KB)
 
-template <typename T8>
-__device__ __forceinline__ void gv_block(const uint8_t* crow, const uint4* lrow, const uint32_t* S,
-                                         const uint16_t* xv, int b, int kq, int C, bool row_ok,
-                                         bool vec_ok, f4_t& acc) {
+// A lane's part of one block: its codes, its row's table and its vector's columns.
+struct GvIn {
+  uint2 cw;
+  uint4 L, xs[4];
+};
+__device__ __forceinline__ GvIn gv_load(const uint8_t* crow, const uint4* lrow, const uint16_t* xv,
+                                        int b, int kq, int C, bool row_ok, bool vec_ok) {
   const int c = b * PB + kq * 32;                // this lane's 32 columns
-  const uint2 cw = row_ok ? *(const uint2*)(crow + b * 32 + kq * 8) : make_uint2(0u, 0u);
-  const uint4 L = row_ok ? lrow[b] : make_uint4(0u, 0u, 0u, 0u);
-  uint4 xs[4];
+  GvIn d;
+  d.cw = row_ok ? *(const uint2*)(crow + b * 32 + kq * 8) : make_uint2(0u, 0u);
+  d.L = row_ok ? lrow[b] : make_uint4(0u, 0u, 0u, 0u);
   if (c + 32 <= C) {                             // all blocks but a ragged last one
     const uint4* xp = (const uint4*)(xv + c);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) xs[k] = vec_ok ? xp[k] : make_uint4(0u, 0u, 0u, 0u);
+    for (int k = 0; k < 4; ++k) d.xs[k] = vec_ok ? xp[k] : make_uint4(0u, 0u, 0u, 0u);
   } else {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -505,20 +513,24 @@ __device__ __forceinline__ void gv_block(const uint8_t* crow, const uint4* lrow,
         const int cc = c + 8 * k + e;
         h[e] = vec_ok && cc < C ? xv[cc] : 0u;
       }
-      xs[k] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16),
-                         h[6] | (h[7] << 16));
+      d.xs[k] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16),
+                           h[6] | (h[7] << 16));
     }
   }
+  return d;
+}
+template <typename T8>
+__device__ __forceinline__ void gv_mul(const GvIn& d, const uint32_t* S, int kq, f4_t& acc) {
   const uint4 s0 = *(const uint4*)(S + kq * 8), s1 = *(const uint4*)(S + kq * 8 + 4);
-  const Planes p = planes_of(L);
+  const Planes p = planes_of(d.L);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const uint32_t w = (k < 2 ? cw.x : cw.y) >> (16 * (k & 1));
+    const uint32_t w = (k < 2 ? d.cw.x : d.cw.y) >> (16 * (k & 1));
     const uint4 sv = k < 2 ? s0 : s1;
     const uint2 a0 = decode4(w & 0xffu, k & 1 ? sv.z : sv.x, p);
     const uint2 a1 = decode4((w >> 8) & 0xffu, k & 1 ? sv.w : sv.y, p);
     acc = mfma_gv<T8>(__builtin_bit_cast(T8, make_uint4(a0.x, a0.y, a1.x, a1.y)),
-                      __builtin_bit_cast(T8, xs[k]), acc);
+                      __builtin_bit_cast(T8, d.xs[k]), acc);
   }
 }
 
@@ -528,7 +540,7 @@ __global__ __launch_bounds__(64 * GV_WAVES) void k_gemv_packed(
     const uint8_t* __restrict__ sal, int R, int C, int nblk, const uint16_t* __restrict__ x,
     int64_t ldx, int nvec, void* __restrict__ y, int64_t ldy, PkEnd end) {
   __shared__ float red[GV_WAVES][16][17];
-  __shared__ __attribute__((aligned(16))) uint32_t Ss[GV_SB * 32];
+  __shared__ __attribute__((aligned(16))) uint32_t Ss[GV_WAVES][64];
   const int r0 = blockIdx.x * 16;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int row = r0 + (lane & 15), kq = lane >> 4, vec = lane & 15;
@@ -536,20 +548,22 @@ __global__ __launch_bounds__(64 * GV_WAVES) void k_gemv_packed(
   const uint8_t* crow = codes + (int64_t)(row_ok ? row : 0) * ldc;
   const uint4* lrow = (const uint4*)(lut + (int64_t)(row_ok ? row : 0) * nblk * 8);
   const uint16_t* xv = x + (int64_t)(vec_ok ? vec : 0) * ldx;
+  uint32_t* const Sw = Ss[wave];
   f4_t acc = {0.f, 0.f, 0.f, 0.f};
-  for (int g = 0; g < nblk; g += GV_SB) {
-    const int n = min(GV_SB, nblk - g);
-    if (g) __syncthreads();                      // the last round's selectors are done with
-    for (int i = threadIdx.x; i < n * 32; i += 64 * GV_WAVES)
-      Ss[i] = sal_bytes(sal[(int64_t)g * 16 + (i >> 1)] >> (4 * (i & 1)));
-    __syncthreads();
-    const int b_end = (int)((int64_t)n * (wave + 1) / GV_WAVES);
-    int b = (int)((int64_t)n * wave / GV_WAVES);
-    for (; b + 1 < b_end; b += 2) {
-      gv_block<T8>(crow, lrow, Ss + b * 32, xv, g + b, kq, C, row_ok, vec_ok, acc);
-      gv_block<T8>(crow, lrow, Ss + b * 32 + 32, xv, g + b + 1, kq, C, row_ok, vec_ok, acc);
-    }
-    if (b < b_end) gv_block<T8>(crow, lrow, Ss + b * 32, xv, g + b, kq, C, row_ok, vec_ok, acc);
+  const int b_end = (int)((int64_t)nblk * (wave + 1) / GV_WAVES);
+  for (int b = (int)((int64_t)nblk * wave / GV_WAVES); b < b_end; b += 2) {
+    const bool two = b + 1 < b_end;
+    const uint32_t sb = lane < 32 || two ? sal[(int64_t)b * 16 + (lane >> 1)] : 0u;
+    const GvIn d0 = gv_load(crow, lrow, xv, b, kq, C, row_ok, vec_ok);
+    GvIn d1;
+    if (two) d1 = gv_load(crow, lrow, xv, b + 1, kq, C, row_ok, vec_ok);
+    // a wavefront's LDS accesses complete in order: no barrier, only the
+    // compiler kept from moving accesses
+    asm volatile("" ::: "memory");
+    Sw[lane] = sal_bytes(sb >> (4 * (lane & 1)));
+    asm volatile("" ::: "memory");
+    gv_mul<T8>(d0, Sw, kq, acc);
+    if (two) gv_mul<T8>(d1, Sw + 32, kq, acc);
   }
   // acc[i] = partial y[vector lane & 15][row r0 + 4 (lane >> 4) + i]
 #pragma unroll
