@@ -17,6 +17,8 @@ no temporary weight is allocated.
 """
 from __future__ import annotations
 
+from operator import itemgetter
+
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
@@ -26,6 +28,7 @@ from ._lib import LINEAR_MAX_EX
 
 GEMV_MAX_TOKENS = 16
 GEMM_MAX_TOKENS = 768
+_parts = itemgetter("codes", "lut", "sal", "bias", "ex_idx")
 
 
 class PackedLinear(nn.Module):
@@ -68,8 +71,12 @@ class PackedLinear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
         x2 = x.reshape(-1, self.in_features)
-        b = self._buffers            # one token's call is host time: no attribute look-ups
-        lut, bias, n_ex = b["lut"], b["bias"], b["ex_idx"].numel()
+        try:                         # one token's call is host time: no attribute look-ups
+            codes, lut, sal, bias, ex_idx = _parts(self._buffers)
+        except KeyError:             # one was assigned as a Parameter, or parametrized
+            codes, lut, sal, bias, ex_idx = (self.codes, self.lut, self.sal, self.bias,
+                                             self.ex_idx)
+        n_ex = ex_idx.numel()
         # product, exceptions, bias and rounding in one kernel: activations and
         # bias in the weights' dtype, few exceptions, a plain [R] bias (one that
         # broadcasts or takes a gradient is added on its own)
@@ -77,16 +84,16 @@ class PackedLinear(nn.Module):
                 and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()
                                       and bias.shape == (self.out_features,)
                                       and not bias.requires_grad))):
-            y = kernels.linear_packed(b["codes"], lut, b["sal"], self.in_features, x2, bias,
+            y = kernels.linear_packed(codes, lut, sal, self.in_features, x2, bias,
                                       self.ex if n_ex else None)
         elif x2.shape[0] <= GEMM_MAX_TOKENS:
             mm = kernels.gemv_packed if x2.shape[0] <= GEMV_MAX_TOKENS else kernels.gemm_packed
-            y = mm(self.codes, self.lut, self.sal, self.in_features, x2, self.ex)
+            y = mm(codes, lut, sal, self.in_features, x2, self.ex)
             y = y.to(x.dtype)
-            if self.bias is not None:
-                y = y + self.bias
+            if bias is not None:
+                y = y + bias
         else:
-            y = F.linear(x2.to(self.lut.dtype), self.weight(), self.bias)
+            y = F.linear(x2.to(lut.dtype), self.weight(), bias)
         return y.reshape(*shape[:-1], self.out_features)
 
     def packed_bytes(self) -> int:

@@ -288,3 +288,23 @@ def test_packed_linear_bias_forms():
     assert torch.equal(y, plain + b)
     y.sum().backward()
     assert torch.equal(b.grad, torch.full_like(b, 20.0))
+
+
+@pytest.mark.parametrize("T", [1, 64, 1024])
+def test_packed_linear_bias_parameter(T):
+    """A bias assigned as a Parameter after construction, on each of the three
+    routes: the product without bias plus that bias, and its gradient."""
+    print(f"packed linear bias parameter T={T}", flush=True)
+    from crb_amd.packed import PackedLinear
+    q, masks = structured(48, 256, seed=6)
+    codes, lut, sal, ex = _k().pack(_q16(q, torch.float16), torch.from_numpy(masks).to(DEV))
+    x = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)).half().to(DEV)
+    b = torch.linspace(-1, 1, 48, device=DEV).half()
+    pl = PackedLinear(codes, lut, sal, 256, torch.zeros_like(b), ex)
+    pl.bias = torch.nn.Parameter(b.clone())
+    y = pl(x)
+    # two fp16 roundings, of a product and of a sum, of at most its size plus 1
+    plain = PackedLinear(codes, lut, sal, 256, None, ex)(x)
+    assert ((y - (plain + b)).abs() <= 2.0 ** -10 * (plain.abs() + 1)).all()
+    y.sum().backward()
+    assert torch.equal(pl.bias.grad, torch.full_like(b, float(T)))
