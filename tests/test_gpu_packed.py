@@ -308,3 +308,29 @@ def test_packed_linear_bias_parameter(T):
     assert ((y - (plain + b)).abs() <= 2.0 ** -10 * (plain.abs() + 1)).all()
     y.sum().backward()
     assert torch.equal(pl.bias.grad, torch.full_like(b, float(T)))
+
+
+@pytest.mark.parametrize("T", [1, 64, 1024])
+def test_packed_linear_bias_transforms(T):
+    """torch.func over the bias, and a dual bias: values of the plain call,
+    tangents and batches kept."""
+    print(f"packed linear bias transforms T={T}", flush=True)
+    import torch.autograd.forward_ad as fwAD
+    from crb_amd.packed import PackedLinear
+    q, masks = structured(48, 256, seed=6)
+    codes, lut, sal, ex = _k().pack(_q16(q, torch.float16), torch.from_numpy(masks).to(DEV))
+    x = torch.randn(T, 256, generator=torch.Generator().manual_seed(T)).half().to(DEV)
+    b, t = torch.linspace(-1, 1, 48, device=DEV).half(), torch.ones(48, device=DEV).half()
+    pl = PackedLinear(codes, lut, sal, 256, b, ex)
+    # two fp16 roundings, of a product and of a sum, of at most its size plus 1
+    bar = 2.0 ** -10 * (pl(x).abs() + 2)
+
+    def f(v):
+        return torch.func.functional_call(pl, {"bias": v}, (x,))
+    y, ty = torch.func.jvp(f, (b,), (t,))
+    assert ((y - pl(x)).abs() <= bar).all() and torch.equal(ty, t.expand(T, 48))
+    ys = torch.func.vmap(f)(torch.stack([b, b]))
+    assert ((ys - pl(x)).abs() <= bar).all()
+    with fwAD.dual_level():
+        y, ty = fwAD.unpack_dual(f(fwAD.make_dual(b, t)))
+        assert ((y - pl(x)).abs() <= bar).all() and torch.equal(ty, t.expand(T, 48))

@@ -74,3 +74,56 @@ def test_parametrized_bias(layer, T):
     nn.utils.parametrize.register_parametrization(pl, "bias", Double())
     x = _x(T)
     assert torch.allclose(pl(x), x @ W.t() + 2, atol=1e-5)
+
+
+@pytest.mark.parametrize("T", TOKENS)
+def test_bias_forward_mode(layer, T):
+    """A bias with a forward-mode tangent keeps it, as a dual tensor and under
+    torch.func.jvp."""
+    import torch.autograd.forward_ad as fwAD
+    make, W, _ = layer
+    b, t = torch.linspace(-1, 1, R), torch.linspace(2, 3, R)
+    pl, x = make(None), _x(T)
+    with fwAD.dual_level():
+        pl.register_buffer("bias", fwAD.make_dual(b, t))
+        y, ty = fwAD.unpack_dual(pl(x))
+        assert torch.allclose(y, x @ W.t() + b, atol=1e-5)
+        assert ty is not None and torch.equal(ty, t.expand(T, R))
+    pl = make(b)
+
+    def f(v):
+        return torch.func.functional_call(pl, {"bias": v}, (x,))
+    y, ty = torch.func.jvp(f, (b,), (t,))
+    assert torch.allclose(y, x @ W.t() + b, atol=1e-5) and torch.equal(ty, t.expand(T, R))
+
+
+@pytest.mark.parametrize("T", TOKENS)
+def test_bias_vmap_and_grad(layer, T):
+    make, W, _ = layer
+    pl, x = make(torch.zeros(R)), _x(T)
+
+    def f(v):
+        return torch.func.functional_call(pl, {"bias": v}, (x,))
+    bs = torch.randn(3, R, generator=torch.Generator().manual_seed(7))
+    y = torch.func.vmap(f)(bs)
+    assert torch.allclose(y, x @ W.t() + bs[:, None], atol=1e-5)
+    g = torch.func.grad(lambda v: f(v).sum())(bs[0])
+    assert torch.equal(g, torch.full((R,), float(T)))
+
+
+class Tagged(torch.Tensor):
+    """A subclass, which torch's add sees and keeps."""
+
+
+def test_bias_subclass_and_negative_view(layer):
+    """A tensor subclass goes to torch's add, and so does a view whose memory
+    holds the negated values."""
+    make, W, calls = layer
+    x = _x(2)
+    b = torch.linspace(-1, 1, R)
+    assert isinstance(make(b.as_subclass(Tagged))(x), Tagged)
+    y = make(torch._neg_view(b))(x)
+    assert calls == ["gemv", "gemv"]
+    assert torch.allclose(y, x @ W.t() - b, atol=1e-5)
+    make(b)(x), make(nn.Parameter(b, requires_grad=False))(x), make(None)(x)
+    assert calls[2:] == ["linear"] * 3
