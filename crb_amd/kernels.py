@@ -510,7 +510,12 @@ def linear_packed(codes: torch.Tensor, lut: torch.Tensor, sal: torch.Tensor, C: 
     the GEMV up to 16 tokens, the GEMM above, bias (in the weights' dtype) and
     exceptions added to the fp32 sums before the one rounding.  At most
     LINEAR_MAX_EX exceptions."""
-    _dev_check(codes, lut, sal, x, bias)
+    if ex is not None and not ex.idx.numel():
+        ex = None
+    dev = codes.get_device()                     # -1 on the CPU
+    if dev < 0 or any(t is not None and t.get_device() != dev
+                      for t in (lut, sal, x, bias, *(ex or ()))):
+        raise _lib.CrbqError("linear_packed: its tensors must live on the GPU, on one device")
     x = _packed_x(x, lut, C, "linear_packed")
     T, R = x.shape[0], codes.shape[0]
     if bias is not None and (bias.dtype != lut.dtype or tuple(bias.shape) != (R,)

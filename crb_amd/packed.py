@@ -88,10 +88,11 @@ class PackedLinear(nn.Module):
                                              self.ex_idx)
         n_ex = ex_idx.numel()
         # product, exceptions, bias and rounding in one kernel: activations and
-        # bias in the weights' dtype, few exceptions, a plain [R] bias (one that
-        # broadcasts or that torch has to see is added on its own)
+        # bias in the weights' dtype, few exceptions, a plain [R] bias on x's
+        # device (one that broadcasts or that torch has to see is added on its own)
         if (x2.shape[0] <= GEMM_MAX_TOKENS and x.dtype == lut.dtype and n_ex <= LINEAR_MAX_EX
-                and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()
+                and (bias is None or (bias.dtype == x.dtype and bias.device == x.device
+                                      and bias.is_contiguous()
                                       and bias.shape == (self.out_features,)
                                       and _plain(bias)))):
             y = kernels.linear_packed(codes, lut, sal, self.in_features, x2, bias,

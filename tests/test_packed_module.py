@@ -127,3 +127,26 @@ def test_bias_subclass_and_negative_view(layer):
     assert torch.allclose(y, x @ W.t() - b, atol=1e-5)
     make(b)(x), make(nn.Parameter(b, requires_grad=False))(x), make(None)(x)
     assert calls[2:] == ["linear"] * 3
+
+
+def test_bias_on_another_device(layer):
+    """torch's add refuses a bias of another device; its address must not
+    reach the kernel (the meta device stands for the other GPU here)."""
+    make, _, calls = layer
+    with pytest.raises(RuntimeError):
+        make(torch.zeros(R, device="meta"))(_x(2))
+    assert calls == ["gemv"]
+
+
+def test_linear_packed_checks_devices():
+    """kernels.linear_packed takes operands of one device only."""
+    from types import SimpleNamespace as NS
+    from crb_amd._lib import CrbqError
+    a, b = (NS(is_cuda=True, get_device=lambda i=i: i, numel=lambda: 1) for i in (0, 1))
+    for bad in range(5):
+        ts = [b if i == bad else a for i in range(5)]
+        with pytest.raises(CrbqError, match="one device"):
+            kernels.linear_packed(ts[0], ts[1], ts[2], C, ts[3], ts[4])
+    ex = kernels.PackedEx(b, b, b)
+    with pytest.raises(CrbqError, match="one device"):
+        kernels.linear_packed(a, a, a, C, a, a, ex)
