@@ -78,8 +78,7 @@ def test_parametrized_bias(layer, T):
 
 @pytest.mark.parametrize("T", TOKENS)
 def test_bias_forward_mode(layer, T):
-    """A bias with a forward-mode tangent keeps it, as a dual tensor and under
-    torch.func.jvp."""
+    """A bias with a forward-mode tangent keeps it."""
     import torch.autograd.forward_ad as fwAD
     make, W, _ = layer
     b, t = torch.linspace(-1, 1, R), torch.linspace(2, 3, R)
@@ -89,16 +88,10 @@ def test_bias_forward_mode(layer, T):
         y, ty = fwAD.unpack_dual(pl(x))
         assert torch.allclose(y, x @ W.t() + b, atol=1e-5)
         assert ty is not None and torch.equal(ty, t.expand(T, R))
-    pl = make(b)
-
-    def f(v):
-        return torch.func.functional_call(pl, {"bias": v}, (x,))
-    y, ty = torch.func.jvp(f, (b,), (t,))
-    assert torch.allclose(y, x @ W.t() + b, atol=1e-5) and torch.equal(ty, t.expand(T, R))
 
 
 @pytest.mark.parametrize("T", TOKENS)
-def test_bias_vmap_and_grad(layer, T):
+def test_bias_vmap(layer, T):
     make, W, _ = layer
     pl, x = make(torch.zeros(R)), _x(T)
 
@@ -107,8 +100,6 @@ def test_bias_vmap_and_grad(layer, T):
     bs = torch.randn(3, R, generator=torch.Generator().manual_seed(7))
     y = torch.func.vmap(f)(bs)
     assert torch.allclose(y, x @ W.t() + bs[:, None], atol=1e-5)
-    g = torch.func.grad(lambda v: f(v).sum())(bs[0])
-    assert torch.equal(g, torch.full((R,), float(T)))
 
 
 class Tagged(torch.Tensor):
