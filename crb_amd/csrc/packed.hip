@@ -821,7 +821,7 @@ __global__ __launch_bounds__(256) void k_gemm_packed_sum(const float* __restrict
                                                          int64_t ldx, void* __restrict__ y,
                                                          int64_t ldy, PkEnd end) {
   const int r = (blockIdx.x * 256 + threadIdx.x) * 4;
-  const bool vec = (R & 3) == 0;
+  const bool vec = (R & 3) == 0 && (((uintptr_t)P) & 15) == 0;   // the caller's workspace
   for (int t = blockIdx.y; t < T; t += gridDim.y) {
     float v[4] = {0.f, 0.f, 0.f, 0.f};
     const float* p = P + (int64_t)t * R + r;

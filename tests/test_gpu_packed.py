@@ -333,3 +333,34 @@ def test_packed_linear_bias_transforms(T):
     with fwAD.dual_level():
         y, ty = fwAD.unpack_dual(f(fwAD.make_dual(b, t)))
         assert ((y - pl(x)).abs() <= bar).all() and torch.equal(ty, t.expand(T, 48))
+
+
+def test_gemm_packed_workspace_alignment():
+    """Split products from a workspace that is only 4-byte aligned: bitwise
+    those from an aligned one."""
+    print("gemm packed workspace alignment", flush=True)
+    from crb_amd import _lib
+    R, C, T = 300, 1920, 17
+    q, masks = structured(R, C, seed=12)
+    codes, lut, sal, _ = _k().pack(_q16(q, torch.float16), torch.from_numpy(masks).to(DEV))
+    x = torch.randn(T, C, generator=torch.Generator().manual_seed(3)).half().to(DEV)
+    lib = _lib.ready(x.device)
+    n = int(lib.crbq_gemm_packed_workspace_size(R, C, T))
+    assert n > 0
+    ws = torch.empty(n // 4 + 4, device=DEV)
+    assert ws.data_ptr() % 16 == 0
+    got = []
+    for off in (0, 1):
+        y = torch.empty(T, R, device=DEV)
+        z = torch.empty(T, R, dtype=torch.float16, device=DEV)
+        w, st = ws[off:].data_ptr(), _lib.stream_of(x)
+        _lib.check(lib.crbq_gemm_packed(codes.data_ptr(), codes.stride(0), lut.data_ptr(),
+                                        sal.data_ptr(), 0, 0, 0, 1, R, C, x.data_ptr(), C, T,
+                                        y.data_ptr(), R, w, n, st), "gemm")
+        _lib.check(lib.crbq_linear_packed(codes.data_ptr(), codes.stride(0), lut.data_ptr(),
+                                          sal.data_ptr(), 0, 0, 0, 1, R, C, x.data_ptr(), C, T, 0,
+                                          z.data_ptr(), R, w, n, st), "linear")
+        got.append((y, z))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert torch.equal(got[0][0].half(), got[0][1])
