@@ -592,7 +592,7 @@ __global__ __launch_bounds__(64 * GV_WAVES) void k_gemv_packed(
 
 // Y[t][r] = sum_c W[r][c] X[t][c] for many tokens (prefill), W packed: each
 // decoded fragment is reused for a tile of up to 16 TG tokens.  A workgroup
-// of GM_WAVES wavefronts covers GM_RT 16-row tiles per wavefront x tt tokens
+// of GM_WAVES wavefronts covers RT 16-row tiles per wavefront x tt tokens
 // (a multiple of 16, up to 16 TG: the tokens are split evenly); per
 // 128-column block each wavefront decodes its rows' 128 columns (lane l: row
 // l & 15 of each tile, columns 32 (l >> 4) .. +31, four 8-column MFMA slices)
@@ -610,18 +610,16 @@ __global__ __launch_bounds__(64 * GV_WAVES) void k_gemv_packed(
 // vector instructions per wavefront and block, half of the wavefronts' time
 // in waits.  Codes and tables of four blocks at a time through LDS (whole
 // lines) measured no faster (85 us at 300 tokens, 34 against 22 at 17).
-constexpr int GM_WAVES = 8, GM_RT = 2;            // wavefronts, row tiles per wavefront
-constexpr int GM_ROWS = 16 * GM_RT * GM_WAVES;
+constexpr int GM_WAVES = 8;
 constexpr int GM_XP = PB + 8;                     // LDS pitch of an X tile row (halves)
 
-template <typename T8, int TG, bool END>
+template <typename T8, int TG, int RT, bool END>
 __global__ __launch_bounds__(64 * GM_WAVES) void k_gemm_packed(
     const uint8_t* __restrict__ codes, int64_t ldc, const uint16_t* __restrict__ lut,
     const uint8_t* __restrict__ sal, int R, int C, int nblk, const uint16_t* __restrict__ x,
     int64_t ldx, int T, int tt, int bps, void* __restrict__ y, int64_t ldy, PkEnd end) {
   __shared__ __attribute__((aligned(16))) uint16_t Xs[2][16 * TG][GM_XP];
   __shared__ __attribute__((aligned(16))) uint32_t Ss[2][32];
-  constexpr int RT = GM_RT;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int r0 = (blockIdx.x * GM_WAVES + wave) * 16 * RT, t0 = blockIdx.y * tt;
   const int b_beg = blockIdx.z * bps, b_end = min(nblk, b_beg + bps);
@@ -869,39 +867,59 @@ __global__ __launch_bounds__(256) void k_gemm_packed_sum(const float* __restrict
 
 // Launch shape of a packed product, a function of the shapes only so that
 // the workspace size is known without a device: 64-token tiles up to 64
-// tokens, else the tokens split evenly over tiles of up to 128, and the
-// number of column splits (of at least 2 blocks) with the least modelled
-// time: rounds of one workgroup per CU, each 5 us and 0.7 + 2.1 tt / 128 us a
-// block, and a sum launch of 3.5 us and the partials written and read at 4
-// TB/s.  Measured against splits to fill the chip once, twice (us): 4096 x
-// 16384 at 300 tokens 74 / 83, at 768 167 / 151, 4096 x 4096 at 300 33 / 34, at
-// 768 57 / 65; against no split, 4096 x 1920 at 64 16 / 26, 1024 x 1024 at 128
-// 18.5 / 24.  One-tile products of up to 8 blocks take no workspace.
+// tokens, else the tokens split evenly over tiles of up to 128; one or two
+// row tiles per wavefront and the number of column splits (of at least 2
+// blocks) with the least modelled time.  Rounds of one workgroup per CU, each
+// 5 us and 0.7 + 2.1 tt / 128 us a block with two row tiles, 3.5 us and 0.5 +
+// 1.8 tt / 128 us with one; a sum launch of 3.5 us and the partials written
+// and read at 4 TB/s.  Two row tiles share every X fragment, which wins where
+// the chip is full; one gives twice the workgroups and a shorter block, which
+// wins where they are few, and is taken if modelled 8 % faster.  Whole linear
+// calls with one / two, each at its own splits (us): 768 x 768 at 17, 64 and
+// 300 tokens 7.7 / 9.1, 9.2 / 10.4, 13.7 / 14.5, 256 x 1024 at 64 11.6 / 17.5,
+// 3072 x 768 at 300 17.8 / 19.2, 4096 x 4096 at 64 and 300 15.4 / 19.5, 41 / 32,
+// 4096 x 16384 at 64 28.8 / 26.9.  Against splits to fill the chip once, twice:
+// 4096 x 16384 at 300 tokens 74 / 83, at 768 167 / 151, 4096 x 4096 at 300 33 /
+// 34, at 768 57 / 65; against no split, 4096 x 1920 at 64 12.1 / 18.3.
+// Products of at most 256 rows, one token tile and 8 blocks take no
+// workspace, as their callers expect (256 x 1024 at 64 tokens 11.6, with
+// splits 8.7).
 struct GmPlan {
-  int tg, tt, ns, bps;
+  int tg, rt, tt, ns, bps;
   int64_t row_tiles, tok_tiles;
 };
 static inline GmPlan gemm_packed_plan(int64_t R, int64_t C, int64_t T) {
   GmPlan p;
   const int64_t nblk = (C + PB - 1) / PB;
   p.tg = T > 64 ? 8 : 4;
-  p.row_tiles = (R + GM_ROWS - 1) / GM_ROWS;
   p.tok_tiles = (T + 16 * p.tg - 1) / (16 * p.tg);
   p.tt = (int)(((T + p.tok_tiles - 1) / p.tok_tiles + 15) / 16 * 16);
   p.tok_tiles = (T + p.tt - 1) / p.tt;
-  const int64_t tiles = p.row_tiles * p.tok_tiles;
-  const double block = 0.7 + 2.1 * p.tt / 128.0, slice = 8.0 * (double)T * (double)R / 4e6;
+  const double slice = 8.0 * (double)T * (double)R / 4e6;
+  const bool none = R <= 256 && p.tok_tiles == 1 && nblk <= 8;
+  const int64_t most = none ? 1 : std::max<int64_t>(1, nblk / 2);
   double best = 0.0;
   p.ns = 0;
-  const int64_t most = tiles == 1 && nblk <= 8 ? 1 : std::max<int64_t>(1, nblk / 2);
-  for (int64_t ns = 1; ns == 1 || (ns <= most && tiles * ns <= 1024); ++ns) {
-    const int64_t per = (nblk + ns - 1) / ns, n = (nblk + per - 1) / per;
-    const double t = (double)((tiles * n + 255) / 256) * (5.0 + block * (double)per) +
-                     (n > 1 ? 3.5 + slice * (double)n : 0.0);
-    if (p.ns == 0 || t < best) {
-      best = t;
-      p.ns = (int)n;
-      p.bps = (int)per;
+  for (int rt = 2; rt >= 1; --rt) {
+    const int64_t rows = 16 * GM_WAVES * rt, row_tiles = (R + rows - 1) / rows;
+    const int64_t tiles = row_tiles * p.tok_tiles;
+    const double wg = rt == 2 ? 5.0 : 3.5;
+    const double block = rt == 2 ? 0.7 + 2.1 * p.tt / 128.0 : 0.5 + 1.8 * p.tt / 128.0;
+    const double less = rt == 2 ? 1.0 : 1.0 / 0.92;
+    int64_t n = 1, per = nblk;
+    while (n == 1 || (n <= most && tiles * n <= 1024)) {
+      const double t = less * ((double)((tiles * n + 255) / 256) * (wg + block * (double)per) +
+                               (n > 1 ? 3.5 + slice * (double)n : 0.0));
+      if (p.ns == 0 || t < best) {
+        best = t;
+        p.rt = rt;
+        p.row_tiles = row_tiles;
+        p.ns = (int)n;
+        p.bps = (int)per;
+      }
+      if (per == 1) break;
+      n = (nblk + per - 2) / (per - 1);        // the fewest splits with fewer blocks each
+      per = (nblk + n - 1) / n;
     }
   }
   return p;
@@ -1023,12 +1041,18 @@ static int gemm_go(const uint8_t* codes, int64_t ldc, const void* lut, const uin
   const bool split = p.ns > 1;
   void* out = split ? ws : y;
   const int64_t ldo = split ? R : ldy;
-#define CRBQ_GM_LAUNCH(T8, TG, E)                                                               \
-  crbq::k_gemm_packed<T8, TG, E><<<grid, 64 * crbq::GM_WAVES, 0, s>>>(                          \
+#define CRBQ_GM_LAUNCH(T8, TG, RT, E)                                                           \
+  crbq::k_gemm_packed<T8, TG, RT, E><<<grid, 64 * crbq::GM_WAVES, 0, s>>>(                      \
       codes, ldc, (const uint16_t*)lut, sal, (int)R, (int)C, nblk, (const uint16_t*)x, ldx,     \
       (int)ntok, p.tt, p.bps, out, ldo, end)
-#define CRBQ_GM_TILE(T8, E) \
-  do { if (p.tg == 8) CRBQ_GM_LAUNCH(T8, 8, E); else CRBQ_GM_LAUNCH(T8, 4, E); } while (0)
+#define CRBQ_GM_TILE(T8, E)                                                               \
+  do {                                                                                    \
+    if (p.rt == 2) {                                                                      \
+      if (p.tg == 8) CRBQ_GM_LAUNCH(T8, 8, 2, E); else CRBQ_GM_LAUNCH(T8, 4, 2, E);       \
+    } else {                                                                              \
+      if (p.tg == 8) CRBQ_GM_LAUNCH(T8, 8, 1, E); else CRBQ_GM_LAUNCH(T8, 4, 1, E);       \
+    }                                                                                     \
+  } while (0)
   if (END && !split) {
     if (dtype == CRBQ_BF16) CRBQ_GM_TILE(b8_t, true); else CRBQ_GM_TILE(h8_t, true);
   } else {

@@ -364,3 +364,33 @@ def test_gemm_packed_workspace_alignment():
     torch.cuda.synchronize()
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     assert torch.equal(got[0][0].half(), got[0][1])
+
+
+@pytest.mark.parametrize("R,C,T,dtype", [
+    (129, 640, 17, torch.float16), (1000, 1000, 129, torch.bfloat16),       # one row tile
+    (33000, 300, 33, torch.float16), (33001, 300, 70, torch.bfloat16),      # two, one launch
+    (8300, 2049, 33, torch.bfloat16), (4099, 2050, 130, torch.float16)])    # two, split sums
+def test_gemm_packed_row_tiles(R, C, T, dtype):
+    """One 16-row tile per wavefront where workgroups are few, two where they
+    fill the chip, at ragged rows, columns and tokens: both products against
+    float64 at the other tests' bars."""
+    print(f"gemm row tiles {R}x{C} T={T} {dtype}", flush=True)
+    q, masks = structured(500, C, seed=R + T, n_odd=0)
+    rep = -(-R // 500)
+    Q = _q16(np.tile(q, (rep, 1))[:R], dtype)
+    Q[::97, 5] = 3.0                     # exceptions, up to 341 rows of them
+    codes, lut, sal, ex = _k().pack(Q, torch.from_numpy(np.tile(masks, (rep, 1))[:R]).to(DEV))
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, C + 40, generator=g).to(dtype).to(DEV)[:, :C]
+    x64, W64 = x.double(), Q.double()
+    ref, scale = x64 @ W64.t(), x64.abs() @ W64.abs().t()
+    y = _k().gemm_packed(codes, lut, sal, C, x, ex)
+    assert ((y.double() - ref).abs() <= 1e-5 * scale + 1e-30).all()
+    n = min(ex.idx.numel(), 256)
+    few = type(ex)(ex.idx[:n], ex.val[:n], ex.delta[:n])
+    b = torch.randn(R, generator=g).to(dtype).to(DEV)
+    z = _k().linear_packed(codes, lut, sal, C, x, b, few)
+    Wf = _k().unpack(codes, lut, sal, C, few).double()
+    ref, scale = x64 @ Wf.t() + b.double(), x64.abs() @ Wf.abs().t() + b.double().abs()
+    half_ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    assert ((z.double() - ref).abs() <= half_ulp * ref.abs() + 1.1e-5 * scale + 2.0 ** -25).all()
