@@ -888,7 +888,9 @@ struct GmPlan {
   int tg, rt, tt, ns, bps;
   int64_t row_tiles, tok_tiles;
 };
-static inline GmPlan gemm_packed_plan(int64_t R, int64_t C, int64_t T) {
+// room: partial slices there is workspace for.
+static inline GmPlan gemm_packed_plan(int64_t R, int64_t C, int64_t T,
+                                      int64_t room = (int64_t)1 << 40) {
   GmPlan p;
   const int64_t nblk = (C + PB - 1) / PB;
   p.tg = T > 64 ? 8 : 4;
@@ -897,7 +899,7 @@ static inline GmPlan gemm_packed_plan(int64_t R, int64_t C, int64_t T) {
   p.tok_tiles = (T + p.tt - 1) / p.tt;
   const double slice = 8.0 * (double)T * (double)R / 4e6;
   const bool none = R <= 256 && p.tok_tiles == 1 && nblk <= 8;
-  const int64_t most = none ? 1 : std::max<int64_t>(1, nblk / 2);
+  const int64_t most = none ? 1 : std::max<int64_t>(1, std::min(nblk / 2, room));
   double best = 0.0;
   p.ns = 0;
   for (int rt = 2; rt >= 1; --rt) {
@@ -923,6 +925,16 @@ static inline GmPlan gemm_packed_plan(int64_t R, int64_t C, int64_t T) {
     }
   }
   return p;
+}
+
+// Partial slices a crbq_gemm_packed call has to bring (crbq.h): splits of at
+// least 8 blocks, as many as keep tiles of 128 rows within 512 workgroups.
+static inline int64_t gemm_packed_least(int64_t R, int64_t C, int64_t T) {
+  const int64_t nblk = (C + PB - 1) / PB, tt = T > 64 ? 128 : 64;
+  const int64_t tiles = ((R + 127) / 128) * ((T + tt - 1) / tt);
+  const int64_t ns = std::max<int64_t>(1, std::min<int64_t>(512 / tiles, nblk / 8));
+  const int64_t per = (nblk + ns - 1) / ns, n = (nblk + per - 1) / per;
+  return n > 1 ? n : 0;
 }
 
 }  // namespace crbq
@@ -1033,9 +1045,13 @@ static int gemm_go(const uint8_t* codes, int64_t ldc, const void* lut, const uin
                    void* y, int64_t ldy, const crbq::PkEnd& end, void* ws, size_t ws_bytes,
                    hipStream_t s) {
   const int nblk = (int)((C + crbq::PB - 1) / crbq::PB);
-  const crbq::GmPlan p = crbq::gemm_packed_plan(R, C, ntok);
+  crbq::GmPlan p = crbq::gemm_packed_plan(R, C, ntok);
   const size_t need = gemm_ws_bytes(p, R, ntok);
-  if (need && (!ws || ws_bytes < need)) return CRBQ_ERR_WORKSPACE;
+  if (need && (!ws || ws_bytes < need)) {
+    const int64_t room = ws ? (int64_t)(ws_bytes / ((size_t)ntok * (size_t)R * sizeof(float))) : 0;
+    if (END || room < crbq::gemm_packed_least(R, C, ntok)) return CRBQ_ERR_WORKSPACE;
+    p = crbq::gemm_packed_plan(R, C, ntok, room);
+  }
   if (p.tok_tiles > 65535) return CRBQ_ERR_ARG;
   const dim3 grid((unsigned)p.row_tiles, (unsigned)p.tok_tiles, (unsigned)p.ns);
   const bool split = p.ns > 1;

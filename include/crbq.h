@@ -327,7 +327,11 @@ int crbq_gemv_packed(const uint8_t* codes, int64_t ldc, const void* lut,
  * column blocks are split over workgroups whose fp32 partials go to the
  * workspace and are summed in split order (deterministic);
  * crbq_gemm_packed_workspace_size(R, C, ntok) bytes (0 when there is no
- * split) depend on the shapes only. */
+ * split) depend on the shapes only.  A smaller workspace (NULL included)
+ * means fewer splits; refused (CRBQ_ERR_WORKSPACE) below n slices of
+ * ntok * R floats, n = ceil(nblk / ceil(nblk / m)) for m = floor(512 / tiles)
+ * but at most floor(nblk / 8), nblk = ceil(C / 128), tiles = 128 rows x 64
+ * tokens each (128 above 64), and n = 0 where that gives one split. */
 size_t crbq_gemm_packed_workspace_size(int64_t R, int64_t C, int64_t ntok);
 int crbq_gemm_packed(const uint8_t* codes, int64_t ldc, const void* lut,
                      const uint8_t* sal, const int64_t* ex_idx, const float* ex_delta,

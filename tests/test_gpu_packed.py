@@ -394,3 +394,40 @@ def test_gemm_packed_row_tiles(R, C, T, dtype):
     ref, scale = x64 @ Wf.t() + b.double(), x64.abs() @ Wf.abs().t() + b.double().abs()
     half_ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
     assert ((z.double() - ref).abs() <= half_ulp * ref.abs() + 1.1e-5 * scale + 2.0 ** -25).all()
+
+
+@pytest.mark.parametrize("R,C,T,least", [(300, 1920, 17, 0), (4096, 1920, 64, 0),
+                                         (1000, 4096, 33, 4)])
+def test_gemm_packed_small_workspace(R, C, T, least):
+    """crbq_gemm_packed with less workspace than it asks for: with the stated
+    minimum (none where splits of 8 blocks are not possible) it runs with
+    fewer splits, below that it is refused; crbq_linear_packed is refused
+    below its full size."""
+    print(f"gemm packed small workspace {R}x{C} T={T}", flush=True)
+    from crb_amd import _lib
+    q, masks = structured(min(R, 300), C, seed=13)
+    rep = -(-R // 300)
+    Q = torch.from_numpy(np.tile(q, (rep, 1))[:R]).to(DEV)
+    codes, lut, sal, _ = _k().pack(Q, torch.from_numpy(np.tile(masks, (rep, 1))[:R]).to(DEV))
+    x = torch.randn(T, C, generator=torch.Generator().manual_seed(3)).half().to(DEV)
+    lib = _lib.ready(x.device)
+    full, slice_ = int(lib.crbq_gemm_packed_workspace_size(R, C, T)), 4 * T * R
+    assert full > least * slice_
+    ws = torch.empty(full, dtype=torch.uint8, device=DEV)
+
+    def call(fn, y, w, n):
+        return fn(codes.data_ptr(), codes.stride(0), lut.data_ptr(), sal.data_ptr(), 0, 0, 0, 1,
+                  R, C, x.data_ptr(), C, T, *((0,) if fn is lib.crbq_linear_packed else ()),
+                  y.data_ptr(), R, w, n, _lib.stream_of(x))
+    ref = x.double() @ Q.double().t()
+    bar = 1e-5 * (x.double().abs() @ Q.double().abs().t()) + 1e-30
+    for n in (least * slice_, full - 1, full):
+        y = torch.empty(T, R, device=DEV)
+        _lib.check(call(lib.crbq_gemm_packed, y, ws.data_ptr() if n else 0, n), "gemm")
+        assert ((y.double() - ref).abs() <= bar).all(), n
+    z = torch.empty(T, R, dtype=torch.float16, device=DEV)
+    refused = -3                          # CRBQ_ERR_WORKSPACE
+    assert call(lib.crbq_linear_packed, z, ws.data_ptr(), full - 1) == refused
+    if least:
+        assert call(lib.crbq_gemm_packed, y, ws.data_ptr(), least * slice_ - 1) == refused
+        assert call(lib.crbq_gemm_packed, y, 0, 0) == refused
