@@ -190,22 +190,25 @@ __device__ __forceinline__ bool last_block(uint32_t* cnt) {
 // k in order, loading all of them before the first add (the partials were
 // written by other workgroups, so every load goes out to memory: one round
 // trip instead of one per batch), then the PARTS subtotals in order.
-// Result in out[0..ncand).
-template <int NK, int PARTS, int GMAX>
+// Result in out[0..ncand).  PAIRS: the partials are added two by two first
+// (2 g and 2 g + 1; GMAX then counts pairs).
+template <int NK, int PARTS, int GMAX, bool PAIRS = false>
 __device__ void reduce_partials(const double* part, int stride, int nwg, int ncand,
                                 double (*red)[NK], double* out) {
   const int t = threadIdx.x, k = t % NK, pp = t / NK;
-  const int G = (nwg + PARTS - 1) / PARTS;
+  const int n = PAIRS ? (nwg + 1) / 2 : nwg;
+  const int G = (n + PARTS - 1) / PARTS;
   double v = 0.0;
   if (k < ncand && pp < PARTS) {
-    double x[GMAX];
+    double x[GMAX], x2[PAIRS ? GMAX : 1];
 #pragma unroll
     for (int j = 0; j < GMAX; ++j) {
-      const int g = pp * G + j;
-      x[j] = (j < G && g < nwg) ? pload(&part[(size_t)g * stride + k]) : 0.0;
+      const int g = pp * G + j, i = PAIRS ? 2 * g : g;
+      x[j] = (j < G && i < nwg) ? pload(&part[(size_t)i * stride + k]) : 0.0;
+      if (PAIRS) x2[j] = (j < G && i + 1 < nwg) ? pload(&part[(size_t)(i + 1) * stride + k]) : 0.0;
     }
 #pragma unroll
-    for (int j = 0; j < GMAX; ++j) v += x[j];
+    for (int j = 0; j < GMAX; ++j) v += PAIRS ? x[j] + x2[j] : x[j];
   }
   if (pp < PARTS) red[pp][k] = v;
   __syncthreads();
@@ -321,8 +324,7 @@ struct ParA {           // a group's fp32 parameters for the residual pass
 // The passes' per-thread elements: element i = tid + 256 k of the
 // workgroup's rows (row r0 + i / nc, column i % nc).  Every load of W is
 // issued before any is used, so the loads overlap instead of each waiting
-// out a memory latency.
-// RPW: rows per workgroup.
+// out a memory latency.  QE: elements per thread.
 template <int QE>
 __device__ __forceinline__ void q_load(const float* __restrict__ W, int64_t ldw, int r0, int r1,
                                        int nc, float (&w)[QE], int (&col)[QE]) {
@@ -862,8 +864,12 @@ __device__ __forceinline__ void wave_prefix(SortedRow& r, float x0, float x1, in
 // fp64 prefix sums of v and v^2; then the workgroup's (row, candidate k)
 // pairs over all its lanes, each two binary searches per group and range
 // sums (group_err1); the last workgroup takes k* = first strict minimum.
-// RPW: rows per workgroup, up to PC_WAVES (the host's search_block).
-template <int RPW>
+// RPW: rows per workgroup, up to PC_WAVES.  GRP: rows that are summed one
+// after the other.  Groups of 8 are added in pairs, here where the workgroup
+// has two and after their trip through memory where it has one, so both give
+// the same bits; with them the grid covers all rows at once (the host's
+// search_block).
+template <int RPW, int GRP>
 __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
     SegSearch seg, int64_t ldw, int R, int nc, int64_t ldu,
     int metric) {
@@ -876,14 +882,15 @@ __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
   __shared__ double e[128];
   __shared__ float pv[NQ];
   __shared__ double errs[PC_WAVES][NQ];
-  __shared__ double acc[NQ];
+  constexpr int NG = RPW / GRP;
+  __shared__ double acc[NG * NQ];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int istar = s.ctrl->istar;
   for (int k = tid; k < NQ; k += 64 * PC_WAVES) {
     pv[k] = np_lerp(s.tval[2 * k], s.tval[2 * k + 1], s.gam[k]);
     if (blockIdx.x == 0) s.pvals[k] = pv[k];
-    acc[k] = 0.0;
   }
+  for (int k = tid; k < NG * NQ; k += 64 * PC_WAVES) acc[k] = 0.0;
   const int c0 = lane, c1 = lane + 64;
   const bool in0 = c0 < nc && s.rank[c0] >= istar, in1 = c1 < nc && s.rank[c1] >= istar;
   float d20 = 1.f, d21 = 1.f;
@@ -910,17 +917,21 @@ __global__ __launch_bounds__(64 * PC_WAVES) void k_phase_c(
       }
     }
     __syncthreads();
-    const int nr = min(RPW, R - r0);
-    for (int k = tid; k < NQ; k += 64 * PC_WAVES) {
-      double v = acc[k];
-      for (int w = 0; w < nr; ++w) v += errs[w][k];
-      acc[k] = v;
+    for (int gk = tid; gk < NG * NQ; gk += 64 * PC_WAVES) {
+      const int g = gk / NQ, k = gk - g * NQ;
+      const int nr = min(RPW, min((g + 1) * GRP, R - r0));
+      double v = acc[gk];
+      for (int w = g * GRP; w < nr; ++w) v += errs[w][k];
+      acc[gk] = v;
     }
   }
   __syncthreads();
-  for (int k = tid; k < NQ; k += 64 * PC_WAVES) pstore(&s.partc[(size_t)blockIdx.x * 96 + k], acc[k]);
+  for (int k = tid; k < NQ; k += 64 * PC_WAVES)
+    pstore(&s.partc[(size_t)blockIdx.x * 96 + k], NG == 2 ? acc[k] + acc[k + (NG - 1) * NQ] : acc[k]);
   if (!last_block(&s.ctrl->cnt[CNT_C])) return;
-  reduce_partials<96, 10, (PX_MAXWG + 9) / 10>(s.partc, 96, gridDim.x, NQ, red, e);
+  constexpr bool pairs = RPW < PC_WAVES;
+  reduce_partials<96, 10, ((pairs ? PX_MAXWG / 2 : PX_MAXWG) + 9) / 10, pairs>(
+      s.partc, 96, gridDim.x, NQ, red, e);
   if (tid < 64) {
     const int am = wave_argmin(e, NQ);
     const int ks = am < 0 ? NQ / 2 : am;                             // :71 median
@@ -1375,18 +1386,26 @@ static int search_block(const SegSearch& seg, int nseg, int64_t ldw, int R, int 
   const int ncand = up_lim - 1;
   const int nwg_cs = (int)std::min<int64_t>(cdiv(R, CS_PH), CS_MAXWG);
   // Few rows leave most CUs idle, and a block is then its launches' latency:
-  // smaller workgroups, the same sums.  Whole loops with this (us per block, before
-  // / after): 256 rows 88 / 70, 768 88 / 73, 1000 88 / 76, 1536 93 / 83, 2048
-  // 96 / 89; 4096 110, unchanged.
-  // Quantile passes: Q_RPW_S rows per workgroup while that gives at most one
-  // workgroup per CU (at 3072 rows 103 against 100, at 4096 119 against 110; 4
-  // rows: 75 at 768 rows, 99 at 2048).
-  const bool qs = R <= 2048;
+  // smaller workgroups.  Whole loops of one weight with this (us per block,
+  // before / after): 256 rows 84 / 66, 768 87 / 72, 1024 88 / 74, 1536 90 / 80,
+  // 2048 92 / 86; 4096 110, unchanged.  A batch multiplies the workgroups, so
+  // the lines below count all its rows.
+  // Quantile passes: Q_RPW_S rows per workgroup up to 1280 rows, and up to
+  // 2048 while a batch has at most 3072 (8 / 32 rows, us per block: 4 x 1024
+  // 103 / 107, 4 x 1280 138 / 141, 2 x 1536 93 / 96, 2 x 2048 102 / 102, 4 x 1536
+  // 145 / 144, 4 x 2048 159 / 153, 1 x 2560 94 / 93; 4 rows, one weight: 75 at
+  // 768 rows, 99 at 2048).  The histograms are counts: the same bits.
+  const bool qs = R <= 1280 || (R <= 2048 && (int64_t)R * nseg <= 3072);
   const int nwg_q = (int)cdiv(R, qs ? Q_RPW_S : Q_RPW);
-  // phase C: 8 rows per workgroup up to 2048 rows, whose 648 (row, candidate)
-  // pairs are one round over its 1024 lanes (16 rows: two) on twice as many
-  // CUs; above, 16 rows, as many workgroups as its partials hold
-  const int rpw = R <= 8 * PX_MAXWG ? PC_WAVES / 2 : PC_WAVES;
+  // phase C: sums of 8 rows added in pairs up to 2048 rows, of 16 above,
+  // whatever the batch, so that a weight's sums are the same alone and in any
+  // batch.  8 rows per workgroup, whose 648 (row, candidate) pairs are one
+  // round over its 1024 lanes (16 rows: two), while the batch's workgroups
+  // are at most one per CU (8 / 16, us per block: 4 x 512 84 / 87, 2 x 1024 83
+  // / 85, 3 x 768 93 / 88, 4 x 1024 112 / 103, 2 x 2048 113 / 102); above 2048
+  // rows as many workgroups as its partials hold
+  const bool pg8 = R <= 8 * PX_MAXWG;
+  const int rpw = (int64_t)R * nseg <= 8 * PX_MAXWG ? PC_WAVES / 2 : PC_WAVES;
   const int nwg_c = (int)std::min<int64_t>(cdiv(R, rpw), PX_MAXWG);
   // phase A: ncg workgroups of up to PR_CW candidates per 64-row group (at
   // least PR_MINW wavefronts: the reduction's 576 threads): as few as hold
@@ -1407,11 +1426,12 @@ static int search_block(const SegSearch& seg, int nseg, int64_t ldw, int R, int 
     k_qlist<Q_RPW><<<dim3(nwg_q, y), 256, 0, st>>>(seg, ldw, R, nc, ldu, metric);
   }
   k_qselect<<<dim3(NT, y), QS_T, 0, st>>>(seg, R, nc);
-  if (rpw == PC_WAVES)
-    k_phase_c<PC_WAVES><<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu, metric);
-  else
-    k_phase_c<PC_WAVES / 2><<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu,
-                                                                      metric);
+#define CRBQ_PC_GO(RPW_, GRP_) \
+  k_phase_c<RPW_, GRP_><<<dim3(nwg_c, y), 64 * PC_WAVES, 0, st>>>(seg, ldw, R, nc, ldu, metric)
+  if (rpw < PC_WAVES) CRBQ_PC_GO(PC_WAVES / 2, PC_WAVES / 2);
+  else if (pg8) CRBQ_PC_GO(PC_WAVES, PC_WAVES / 2);
+  else CRBQ_PC_GO(PC_WAVES, PC_WAVES);
+#undef CRBQ_PC_GO
   CRBQ_LAUNCH_CHECK();
   return CRBQ_OK;
 }

@@ -78,6 +78,31 @@ def test_batched_matches_one_call_per_sublayer(method, partition, gptq, n, R, C,
         assert torch.equal(Wb[i][:, C:], base[i][:, C:]), i
 
 
+@pytest.mark.parametrize("n,R", [(4, 512), (3, 683), (4, 1024), (3, 1001), (2, 1992), (2, 2041),
+                                 (2, 2048), (3, 1281), (2, 2049)])
+def test_batched_row_counts(n, R):
+    """Row counts around the search's workgroup sizes, which depend on the
+    batch (8 or 16 rows per phase C workgroup with partial sums of 8, 8 or 32
+    rows per quantile workgroup; a last workgroup with an empty second half at
+    1992): every weight bitwise as alone, traces included."""
+    from crb_amd import _lib, kernels
+    print(f"batched rows n={n} R={R}", flush=True)
+    C = 256
+    p = _lib.params("crb")
+    Us = [_factor(C, R)] * n
+    base = _weights(n, R, C, C, R + n)
+    ref = _one_by_one(base, C, Us, p)
+    Ws = [base[i].clone() for i in range(n)]
+    Ls = [torch.zeros(R, device=DEV) for _ in range(n)]
+    masks, traces = kernels.fasterquant_blocks_batched(Ws, Us[0], p, Ls, want_masks=True,
+                                                       want_traces=True)
+    torch.cuda.synchronize()
+    for i in range(n):
+        W, L, m, t = ref[i]
+        assert torch.equal(Ws[i], W) and torch.equal(Ls[i], L) and torch.equal(masks[i], m), i
+        assert traces[i] == t, i
+
+
 def test_batched_single_segment_and_argument_checks():
     from crb_amd import _lib, kernels
     print("batched nseg=1 and argument checks", flush=True)
