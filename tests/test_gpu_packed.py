@@ -431,3 +431,25 @@ def test_gemm_packed_small_workspace(R, C, T, least):
     if least:
         assert call(lib.crbq_gemm_packed, y, ws.data_ptr(), least * slice_ - 1) == refused
         assert call(lib.crbq_gemm_packed, y, 0, 0) == refused
+
+
+@pytest.mark.parametrize("R,C", [(1, 1), (5, 8), (1025, 9), (2047, 17), (515, 24), (257, 65),
+                                 (131, 136), (67, 1032), (9, 2049), (70_000_003, 8)])
+def test_unpack_thread_shapes(R, C):
+    """Unpack against the format statement where its threads change shape (as
+    many along a row as it has chunks of 8 columns, the rest down the rows),
+    and at more rows than a launch has four-row workgroups."""
+    print(f"unpack shapes {R}x{C}", flush=True)
+    nblk = -(-C // 128)
+    g = torch.Generator(device=DEV).manual_seed(R % 1000 + C)
+    codes = torch.randint(0, 256, (R, nblk * 32), device=DEV, generator=g, dtype=torch.uint8)
+    lut = torch.randint(-32768, 32767, (R, nblk, 8), device=DEV, generator=g,
+                        dtype=torch.int16).view(torch.float16)
+    sal = torch.randint(0, 256, (nblk, 16), device=DEV, generator=g, dtype=torch.uint8)
+    Q = _k().unpack(codes, lut, sal, C).view(torch.int16)
+    bits = lut.view(torch.int16)
+    for c in range(C):
+        code = (codes[:, c // 4] >> (2 * (c % 4))) & 3
+        s = int(sal[c // 128, (c % 128) // 8]) >> (c % 8) & 1
+        want = bits[:, c // 128].gather(1, (code.long() + 4 * s)[:, None])[:, 0]
+        assert torch.equal(Q[:, c], want), c
