@@ -92,19 +92,22 @@ __device__ __forceinline__ void pack_block(const uint16_t* __restrict__ Q, int64
     int cand[NDV], cnt[NDV], nd = 0, prev = -1;
 #pragma unroll
     for (int k = 0; k < NDV; ++k) {
+      cand[k] = 0x10000;
+      cnt[k] = 0;
+    }
+#pragma unroll
+    for (int k = 0; k < NDV; ++k) {
       int m = 0x10000;
 #pragma unroll
       for (int s = 0; s < 2; ++s)
         if (grp[s] == G && key[s] > prev) m = min(m, key[s]);
-      m = wave_min_i(m);
+      m = __builtin_amdgcn_readfirstlane(wave_min_i(m));
+      if (m >= 0x10000) break;
       cand[k] = m;
-      cnt[k] = 0;
-      if (m < 0x10000) {
-        cnt[k] = __popcll(__ballot(grp[0] == G && key[0] == m)) +
-                 __popcll(__ballot(grp[1] == G && key[1] == m));
-        nd = k + 1;
-        prev = m;
-      }
+      cnt[k] = __popcll(__ballot(grp[0] == G && key[0] == m)) +
+               __popcll(__ballot(grp[1] == G && key[1] == m));
+      nd = k + 1;
+      prev = m;
     }
     // keep the cap most frequent (ties: smaller key), in ascending key order
     bool keep[NDV];
@@ -187,11 +190,15 @@ __device__ __forceinline__ us2_t row_pk_min(us2_t v) {
 // group 3, so each group's table is its smallest and largest value (kept as
 // the minima of key and ~key in the halves of one register) and, for group
 // 3, the smallest and largest of what is left; a block row with an element
-// outside those goes through pack_block, one wavefront each.  Bound by
-// issue (about 330 instructions per 4 block rows): with the host's part 88
-// us for 4096 x 4096 and 191 for 4096 x 16384, against 357 and 1254 with one
-// wavefront per block row and eight minimum searches per group.
-__global__ __launch_bounds__(256) void k_pack(const uint16_t* __restrict__ Q, int64_t ldq,
+// outside those goes through pack_block, the workgroup's in turn over its
+// wavefronts (768 x 768 with 500 exceptions 104 us; each wavefront its own,
+// 112; 16 wavefronts per workgroup 101, but 295 for 4096 x 16384 without
+// any).  Bound by issue (about 330 instructions per 4 block rows): with the
+// host's part 88 us for 4096 x 4096 and 196 for 4096 x 16384, against 357
+// and 1254 with one wavefront per block row and eight minimum searches per
+// group.
+constexpr int PK_WAVES = 4;
+__global__ __launch_bounds__(64 * PK_WAVES) void k_pack(const uint16_t* __restrict__ Q, int64_t ldq,
                                               const uint8_t* __restrict__ M, int64_t ldm,
                                               int R, int C, int nblk, bool bf16,
                                               uint8_t* __restrict__ codes, int64_t ldc,
@@ -201,7 +208,8 @@ __global__ __launch_bounds__(256) void k_pack(const uint16_t* __restrict__ Q, in
                                               uint16_t* __restrict__ ex_val,
                                               float* __restrict__ ex_delta, int ex_cap,
                                               int* ex_count, int* status) {
-  const int64_t w = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  __shared__ unsigned slow4[PK_WAVES];
+  const int64_t w = (int64_t)blockIdx.x * (4 * PK_WAVES) + (threadIdx.x >> 4);
   const bool live = w < (int64_t)R * nblk;
   const int r = live ? (int)(w / nblk) : 0, b = live ? (int)(w - (int64_t)r * nblk) : 0;
   const int l16 = threadIdx.x & 15;
@@ -306,11 +314,19 @@ __global__ __launch_bounds__(256) void k_pack(const uint16_t* __restrict__ Q, in
   if (!live) err = 0;
   err = wave_or_i(err);
   if (lane == 0 && err) atomicOr(status, err);
-  if (sm) {                                  // uniform: the wavefront's block rows in turn
+  // block rows with exceptions: the workgroup's, over its wavefronts in turn
+  auto any16 = [&](int k) { return (unsigned)(((sm >> (16 * k)) & 0xffffull) != 0) << k; };
+  if (lane == 0) slow4[threadIdx.x >> 6] = any16(0) | any16(1) | any16(2) | any16(3);
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  int k = 0;
 #pragma unroll 1
-    for (int k = 0; k < 4; ++k) {
-      if (((sm >> (16 * k)) & 0xffffull) == 0) continue;
-      const int rr = __shfl(r, 16 * k, CRBQ_WAVE), bb = __shfl(b, 16 * k, CRBQ_WAVE);
+  for (int q = 0; q < PK_WAVES; ++q) {
+    unsigned todo = __builtin_amdgcn_readfirstlane(slow4[q]);
+    for (; todo; todo &= todo - 1, ++k) {
+      if (k % PK_WAVES != wave) continue;
+      const int64_t wi = (int64_t)blockIdx.x * (4 * PK_WAVES) + 4 * q + __builtin_ctz(todo);
+      const int rr = (int)(wi / nblk), bb = (int)(wi - (int64_t)rr * nblk);
       pack_block(Q, ldq, M, ldm, rr, bb, C, nblk, bf16, codes, ldc, lut, ex_idx, ex_val, ex_delta,
                  ex_cap, ex_count, status);
     }
@@ -963,7 +979,8 @@ extern "C" int crbq_pack(const void* Q, int dtype, int64_t R, int64_t C, int64_t
   crbq::k_zero_status<<<1, 1, 0, s>>>(status, ex_count);
   CRBQ_LAUNCH_CHECK();
   const int64_t rows = R * nblk;
-  crbq::k_pack<<<(unsigned)((rows + 15) / 16), 256, 0, s>>>(
+  crbq::k_pack<<<(unsigned)((rows + 4 * crbq::PK_WAVES - 1) / (4 * crbq::PK_WAVES)),
+                 64 * crbq::PK_WAVES, 0, s>>>(
       (const uint16_t*)Q, ldq, masks, ldm, (int)R, (int)C, (int)nblk, dtype == CRBQ_BF16, codes,
       ldc, (uint16_t*)lut, sal, ex_idx, (uint16_t*)ex_val, ex_delta, ex_cap, ex_count, status);
   CRBQ_LAUNCH_CHECK();

@@ -453,3 +453,20 @@ def test_unpack_thread_shapes(R, C):
         s = int(sal[c // 128, (c % 128) // 8]) >> (c % 8) & 1
         want = bits[:, c // 128].gather(1, (code.long() + 4 * s)[:, None])[:, 0]
         assert torch.equal(Q[:, c], want), c
+
+
+@pytest.mark.parametrize("R,C,n_odd", [(20, 300, 2000), (7, 1000, 12), (33, 128, 33)])
+def test_pack_many_exceptions(R, C, n_odd):
+    """Block rows with exceptions, from a few of a workgroup's 16 to all of
+    them, one wavefront each in turn: against the format statement."""
+    print(f"pack many exceptions {R}x{C} odd={n_odd}", flush=True)
+    q, masks = structured(R, C, seed=R, n_odd=n_odd)
+    codes, lut, sal, ex = _k().pack(_q16(q, torch.float16), torch.from_numpy(masks).to(DEV),
+                                    ex_cap=R * C)
+    rc, rl, rs, rex, st = pack_ref(q.view(np.uint16), masks, ex_cap=R * C)
+    assert st == 0 and np.array_equal(codes.cpu().numpy(), rc)
+    assert np.array_equal(lut.cpu().view(torch.int16).numpy().view(np.uint16), rl)
+    assert np.array_equal(sal.cpu().numpy(), rs)
+    assert np.array_equal(ex.idx.cpu().numpy(), rex[0])
+    assert np.array_equal(ex.val.cpu().view(torch.int16).numpy().view(np.uint16), rex[1])
+    assert np.array_equal(ex.delta.cpu().numpy(), rex[2])
