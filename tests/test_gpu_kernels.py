@@ -421,6 +421,27 @@ def test_hessian_small_tiles(dtype, T, C, ldx):
     assert (torch.tril(S1, -1) == torch.tril(torch.full_like(S1, 0.5), -1)).all()
 
 
+@pytest.mark.parametrize("T,C,ldx", [(1, 7, 7), (70, 250, 250), (64, 9, 11), (3, 65, 66),
+                                     (131, 250, 257)])
+def test_hessian_small_tiles_row_ends(T, C, ldx):
+    """Channel counts that are no multiple of 8: the 64 x 64 tiles' loads run
+    past a row's end into what follows in X (here NaN), which reaches no
+    output; bitwise the channel-major kernel's sums."""
+    print(f"hessian small row ends T={T} C={C} ldx={ldx}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + C)
+    buf = torch.full((T, ldx), float("nan"), device=DEV, dtype=torch.float16)
+    X = buf[:, :C]
+    X.copy_(torch.randn(T, C, device=DEV, generator=g))
+    S1 = torch.full((C, C), 0.5, device=DEV)
+    _k().hessian_accum(X, S1)
+    Xt = _k().hessian_cm_store(T, C, torch.float16, DEV)
+    _k().hessian_transpose(X.contiguous(), Xt, 0)
+    S2 = torch.full((C, C), 0.5, device=DEV)
+    _k().hessian_accum_cm(Xt, T, C, S2)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.triu(S1), torch.triu(S2))
+
+
 def test_hessian_matches_reference_add_batch():
     """Incremental rescale of bigptq.py:50-53 vs. one 2/n scaling."""
     print("hessian add_batch", flush=True)
