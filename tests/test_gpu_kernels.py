@@ -184,9 +184,10 @@ def _hess_want(X, S0):
 @pytest.mark.parametrize("T,C,ldx", [(300, 200, 200), (1000, 384, 392), (77, 8, 13),
                                      (8192, 520, 520)])
 def test_hessian_token_major_path(dtype, T, C, ldx):
-    """The in-place SYRK taken when the workspace cannot hold the
-    channel-major copy: NULL workspace, and a workspace sized for the split
-    partials only."""
+    """Calls whose workspace cannot hold the channel-major copy: NULL
+    workspace, and a workspace sized for the split partials only.  At these
+    sizes they run on 64 x 64 tiles (k_syrk16s); the in-place SYRK k_syrk16p
+    has test_hessian_large_in_place."""
     print(f"hessian token-major {dtype} T={T} C={C} ldx={ldx}", flush=True)
     from crb_amd import _lib
     lib = _lib.load()
@@ -214,7 +215,9 @@ def test_hessian_token_major_path(dtype, T, C, ldx):
 def test_hessian_channel_major_passes(dtype, T, C, ldx, pass_tok, monkeypatch):
     """Inputs longer than one transposed pass run in several passes (the pass
     length is lowered through CRBQ_XT_PASS_TOKENS); ragged last pass, C not a
-    multiple of the 256-channel tile, strided rows."""
+    multiple of the 256-channel tile, strided rows.  At these sizes a pass
+    runs on 64 x 64 tiles straight from X; transposed passes have
+    test_hessian_large_passes."""
     print(f"hessian passes {dtype} T={T} C={C} pass={pass_tok}", flush=True)
     from crb_amd import _lib
     lib = _lib.load()
@@ -278,7 +281,8 @@ def test_hessian_channel_major_store(dtype, C, chunks):
 def test_hessian_token_major_stages(dtype, T, C, ldx):
     """C a multiple of 256 with 16-byte aligned rows: the SYRK stages the
     token-major X as it is and reads its MFMA operands with LDS transpose
-    reads.  Bitwise the sums of the channel-major path (crbq_hessian_transpose
+    reads (k_syrk16k, k_syrk16k_pers; up to 512 channels k_syrk16s, which does
+    the same on 64 x 64 tiles).  Bitwise the sums of the channel-major path (crbq_hessian_transpose
     + crbq_hessian_accum_cm, same token splits) on the same tokens, and
     against float64: ragged token counts (rows past ntok read as zeros),
     strided rows, the launched grid, the persistent kernel (C = 8192) and
@@ -319,9 +323,10 @@ def test_hessian_token_major_stages(dtype, T, C, ldx):
 @pytest.mark.parametrize("T,C,ldx", [(300, 512, 513), (5000, 256, 260)])
 def test_hessian_token_major_unaligned(dtype, T, C, ldx):
     """C a multiple of 256 but rows that cannot be staged with 16-byte loads
-    (odd or non-multiple-of-8 row stride): crbq_hessian_workspace_size then
-    holds only the split partials, so the SYRK transposes in registers
-    (k_syrk16p); against float64."""
+    (odd or non-multiple-of-8 row stride), with a workspace that holds only
+    the split partials: these sizes run on 64 x 64 tiles with unaligned loads
+    (k_syrk16s), larger ones transpose in registers (k_syrk16p,
+    test_hessian_large_in_place); against float64."""
     print(f"hessian token-major unaligned {dtype} T={T} C={C} ldx={ldx}", flush=True)
     from crb_amd import _lib
     lib = _lib.load()
@@ -337,6 +342,101 @@ def test_hessian_token_major_unaligned(dtype, T, C, ldx):
     Xd = X.double()
     want = torch.triu(Xd.t() @ Xd + 0.25)
     assert float((torch.triu(S.double()) - want).norm() / want.norm()) < 1e-5
+
+
+def _splits_and_small(T, C):
+    """The 16-bit SYRK's dispatch (choose_splits and syrk16_small in
+    hessian.hip) restated: token splits of the 256 x 256 tiles, and whether
+    the call runs on 64 x 64 tiles instead."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tpad, n256, n64 = -(-T // 64) * 64, -(-C // 256), -(-C // 64)
+    tiles, best = n256 * (n256 + 1) // 2, None
+    for ns in range(1, 17):
+        if ns > 1 and tpad // ns < 2048:
+            break
+        t = (-(-tiles * ns // cus) * -(-tpad // ns) * 2.0 * 256 * 256 / (4096.0 * 2.4e9 * 0.6)
+             + (2.0 * ns * C * C * 4.0 / 5e12 if ns > 1 else 0.0))
+        if best is None or t < best[0]:
+            best = t, ns
+    ns = best[1]
+    stages = -(-(tpad // 64) // ns)
+    ts = 8.0 + max(n64 * (n64 + 1) // 2 * tpad * 256.0 / 10e6, 0.3 * stages)
+    return ns, ts <= 26.0 + 1.75 * stages * -(-tiles * ns // cus)
+
+
+def _rand_x(T, C, ldx, dtype):
+    g = torch.Generator(device=DEV).manual_seed(T + 3 * C + ldx)
+    return (torch.randn(T, ldx, device=DEV, generator=g) *
+            torch.exp(torch.randn(ldx, device=DEV, generator=g))).to(dtype)[:, :C]
+
+
+def _rel_hess(S, X, S0):
+    Xd = X.double()
+    want = torch.triu(Xd.t() @ Xd + S0)
+    return float((torch.triu(S.double()) - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,C,ldx,slices", [
+    (4203, 2312, 2312, 0), (16500, 2056, 2056, 4),          # 16-byte loads: one split, four
+    (4203, 2560, 2563, 0), (16500, 1536, 1541, 5), (16500, 2056, 2059, 4)])
+def test_hessian_large_in_place(dtype, T, C, ldx, slices):
+    """The in-place SYRK k_syrk16p, at sizes that 256 x 256 tiles keep: a
+    workspace without room for the channel-major copy, NULL (one split) or
+    `slices` split partials, rows that allow 16-byte loads and rows that do
+    not; against float64, and the same bits again."""
+    print(f"hessian large in place {dtype} T={T} C={C} ldx={ldx} slices={slices}", flush=True)
+    ns, small = _splits_and_small(T, C)
+    nb = slices * C * C * 4
+    assert not small and nb < -(-C // 256) * 256 * (-(-T // 64) * 64) * 2
+    assert slices == 0 or 1 < slices <= ns
+    X = _rand_x(T, C, ldx, dtype)
+    S = torch.full((C, C), 0.25, device=DEV)
+    _accum_raw(X, S, nb)
+    assert _rel_hess(S, X, 0.25) < 1e-5
+    S2 = torch.full((C, C), 0.25, device=DEV)
+    _accum_raw(X, S2, nb)
+    assert torch.equal(torch.triu(S), torch.triu(S2))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,C,ldx", [(6203, 2056, 2056), (6203, 2056, 2059)])
+def test_hessian_large_passes(dtype, T, C, ldx, monkeypatch):
+    """Several transposed passes at a size that 256 x 256 tiles keep (aligned
+    rows and not): bitwise the passes' token slices one call after the other,
+    whose own 64 x 64 tiles give the same sums, and against float64."""
+    print(f"hessian large passes {dtype} T={T} C={C} ldx={ldx}", flush=True)
+    from crb_amd import _lib
+    assert not _splits_and_small(T, C)[1] and _splits_and_small(2496, C)[1]
+    lib = _lib.load()
+    X = _rand_x(T, C, ldx, dtype)
+    monkeypatch.setenv("CRBQ_XT_PASS_TOKENS", "2500")
+    nb = lib.crbq_hessian_workspace_size(T, C)
+    S, S2 = (torch.ones(C, C, device=DEV) for _ in range(2))
+    _accum_raw(X, S, nb)
+    for t0 in range(0, T, 2496):
+        _accum_raw(X[t0:t0 + 2496], S2, nb)
+    assert torch.equal(torch.triu(S), torch.triu(S2))
+    assert _rel_hess(S, X, 1.0) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,C,ldx", [(6203, 2560, 2568), (12301, 1536, 1536)])
+def test_hessian_large_launched_grid(dtype, T, C, ldx):
+    """Token-major stages on the launched grid of 256 x 256 tiles with several
+    token splits: bitwise the channel-major kernel's sums, and against
+    float64."""
+    print(f"hessian large grid {dtype} T={T} C={C} ldx={ldx}", flush=True)
+    ns, small = _splits_and_small(T, C)
+    assert ns > 1 and not small
+    X = _rand_x(T, C, ldx, dtype)
+    S1, S2 = (torch.full((C, C), 0.5, device=DEV) for _ in range(2))
+    _k().hessian_accum(X, S1)
+    Xt = _k().hessian_cm_store(T, C, dtype, DEV)
+    _k().hessian_transpose(X, Xt, 0)
+    _k().hessian_accum_cm(Xt, T, C, S2)
+    assert torch.equal(torch.triu(S1), torch.triu(S2))
+    assert _rel_hess(S1, X, 0.5) < 1e-5
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
