@@ -193,10 +193,10 @@ __device__ __forceinline__ us2_t row_pk_min(us2_t v) {
 // outside those goes through pack_block, the workgroup's in turn over its
 // wavefronts (768 x 768 with 500 exceptions 104 us; each wavefront its own,
 // 112; 16 wavefronts per workgroup 101, but 295 for 4096 x 16384 without
-// any).  Bound by issue (about 330 instructions per 4 block rows): with the
-// host's part 88 us for 4096 x 4096 and 196 for 4096 x 16384, against 357
-// and 1254 with one wavefront per block row and eight minimum searches per
-// group.
+// any).  Bound by issue (784 vector instructions per 4 block rows, 84 % of
+// the time busy): with the host's part 88 us for 4096 x 4096, 45 of them the
+// kernel, and 196 for 4096 x 16384, against 357 and 1254 with one wavefront
+// per block row and eight minimum searches per group.
 constexpr int PK_WAVES = 4;
 __global__ __launch_bounds__(64 * PK_WAVES) void k_pack(const uint16_t* __restrict__ Q, int64_t ldq,
                                               const uint8_t* __restrict__ M, int64_t ldm,
@@ -352,8 +352,8 @@ __device__ __forceinline__ Planes planes_of(uint4 L) {
 __device__ __forceinline__ uint32_t sal_bytes(uint32_t n) {
   return ((n & 15u) * 0x00204081u & 0x01010101u) << 2;
 }
-// Weights of code byte c (bits 0-7 of c, what is above is dropped by the
-// mask) and salient selector S as two 32-bit pairs.
+// Weights of code byte c (0-255: a bit above would reach code 1) and salient
+// selector S as two 32-bit pairs.
 __device__ __forceinline__ uint2 decode4(uint32_t c, uint32_t S, const Planes& t) {
   const uint32_t x = (c << 12) | c, y = (x << 6) | x;    // code j at bits 8 j
   const uint32_t sel = (y & 0x03030303u) | S;

@@ -157,7 +157,7 @@ def test_gemv_against_float64(R, C, dtype, nvec):
 def test_gemm_against_float64(R, C, T, dtype):
     """crbq_gemm_packed against float64 products of the unpacked weights,
     same bar as the GEMV; the split-K and single-pass launches are both
-    covered (the split depends on R x T tiles)."""
+    covered (the split depends on the shapes)."""
     print(f"gemm {R}x{C} T={T} {dtype}", flush=True)
     from crb_amd import _lib
     q, masks = structured(R, C, seed=5 * R + C, n_odd=R // 8)
@@ -173,7 +173,8 @@ def test_gemm_against_float64(R, C, T, dtype):
     scale = x64.abs() @ W64.abs().t()
     err = (y.double().cpu() - ref).abs()
     assert (err <= 1e-5 * scale + 1e-30).all(), float((err / scale.clamp_min(1e-30)).max())
-    # the header's rule: floor(512 / tiles) splits of >= 8 blocks each
+    # which of these shapes split: those for which the header's minimum asks
+    # for partials (the number of splits comes from the modelled time)
     tiles = -(-R // 128) * -(-T // (128 if T > 64 else 64))
     split = min(512 // tiles, -(-C // 128) // 8) > 1
     lib = _lib.load()
