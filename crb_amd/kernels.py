@@ -513,8 +513,9 @@ def linear_packed(codes: torch.Tensor, lut: torch.Tensor, sal: torch.Tensor, C: 
     if ex is not None and not ex.idx.numel():
         ex = None
     dev = codes.get_device()                     # -1 on the CPU
-    if dev < 0 or any(t is not None and t.get_device() != dev
-                      for t in (lut, sal, x, bias, *(ex or ()))):
+    if (dev < 0 or lut.get_device() != dev or sal.get_device() != dev or x.get_device() != dev
+            or (bias is not None and bias.get_device() != dev)
+            or (ex is not None and any(t.get_device() != dev for t in ex))):
         raise _lib.CrbqError("linear_packed: its tensors must live on the GPU, on one device")
     x = _packed_x(x, lut, C, "linear_packed")
     T, R = x.shape[0], codes.shape[0]

@@ -20,9 +20,9 @@ from __future__ import annotations
 from operator import itemgetter
 
 import torch
+import torch.autograd.forward_ad as fwad
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.autograd.forward_ad import unpack_dual
 
 from . import kernels
 from ._lib import LINEAR_MAX_EX
@@ -31,14 +31,15 @@ GEMV_MAX_TOKENS = 16
 GEMM_MAX_TOKENS = 768
 _parts = itemgetter("codes", "lut", "sal", "bias", "ex_idx")
 _wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+_PLAIN = frozenset((torch.Tensor, nn.Parameter))
 
 
 def _plain(b: torch.Tensor) -> bool:
     """Whether a kernel may read b's memory in the place of torch's add: no
     gradient, no forward-mode tangent, no torch.func wrapper, no subclass, no
     negated view."""
-    return (type(b) in (torch.Tensor, nn.Parameter) and not b.requires_grad
-            and not b.is_neg() and not _wrapped(b) and unpack_dual(b).tangent is None)
+    return (type(b) in _PLAIN and not b.requires_grad and not b.is_neg() and not _wrapped(b)
+            and (fwad._current_level < 0 or fwad.unpack_dual(b).tangent is None))
 
 
 class PackedLinear(nn.Module):
@@ -88,11 +89,10 @@ class PackedLinear(nn.Module):
                                              self.ex_idx)
         n_ex = ex_idx.numel()
         # product, exceptions, bias and rounding in one kernel: activations and
-        # bias in the weights' dtype, few exceptions, a plain [R] bias on x's
-        # device (one that broadcasts or that torch has to see is added on its own)
+        # bias in the weights' dtype, few exceptions, a plain [R] bias (one that
+        # broadcasts or that torch has to see is added on its own)
         if (x2.shape[0] <= GEMM_MAX_TOKENS and x.dtype == lut.dtype and n_ex <= LINEAR_MAX_EX
-                and (bias is None or (bias.dtype == x.dtype and bias.device == x.device
-                                      and bias.is_contiguous()
+                and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()
                                       and bias.shape == (self.out_features,)
                                       and _plain(bias)))):
             y = kernels.linear_packed(codes, lut, sal, self.in_features, x2, bias,
