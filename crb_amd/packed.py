@@ -7,13 +7,14 @@ row, one salient-column bitmap per block; the format is described in
 include/crbq.h) and multiplies with them directly: up to 16 tokens per call
 through the packed GEMV (MFMA on weights decoded in registers), up to 768
 through the packed GEMM (each decoded fragment reused for up to 128 tokens),
-with bias and rounding in the same kernels, and larger batches, where the
-product is compute-bound, by unpacking into a temporary dense weight for the
-dense GEMM.  Packed / through the dense weight on MI355X, us: 4096 x 16384 at
-256 / 512 / 768 / 1024 tokens 63 / 99, 104 / 120, 158 / 138, 183 / 165; 16384 x
-4096 60 / 71, 94 / 90, 168 / 110, 185 / 130; 4096 x 4096 29 / 37, 40 / 40, 56 /
-43, 60 / 50; 1024 x 4096 21 / 37, 24 / 36, 26 / 36, 29 / 36.  Up to 768 tokens
-no temporary weight is allocated.
+with bias and rounding in the same kernels, and larger batches by unpacking
+into a temporary dense weight for the dense GEMM.  The second limit bounds
+memory (up to 768 tokens no temporary weight is allocated); in time the dense
+route wins from about 512 tokens on the larger layers.  Packed / through the
+dense weight on MI355X, us: 4096 x 16384 at 256 / 512 / 768 / 1024 tokens 62 /
+94, 101 / 120, 156 / 138, 182 / 161; 16384 x 4096 61 / 70, 86 / 89, 164 / 109,
+175 / 131; 4096 x 4096 29 / 32, 39 / 39, 56 / 44, 60 / 49; 1024 x 4096 20 / 32,
+23 / 32, 26 / 32, 29 / 32; 768 x 768 16 / 32, 16 / 32, 16 / 32, 18 / 32.
 """
 from __future__ import annotations
 
