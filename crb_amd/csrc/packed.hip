@@ -17,6 +17,7 @@
 // for non-salient weights and rank (0..3) for salient ones: 3 bits per
 // weight instead of 16, and unpacking reproduces the weights bit for bit.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -723,24 +724,33 @@ __global__ __launch_bounds__(64 * GM_WAVES) void k_gemm_packed(
   // Block b: multiply its fragments while block b + 1's are decoded, a part
   // with each token group (decoding at the top of a block, where the barrier
   // has just lined the wavefronts up, left the matrix units idle meanwhile);
-  // X is loaded one block ahead, codes, tables and salient bits two.
-  for (int b = b_beg; b < b_end; ++b) {
+  // X is loaded one block ahead, codes, tables and salient bits two.  The
+  // last block stands by itself, with nothing to load or decode behind it:
+  // 64 x 64 at 64 tokens 5.0 us to 4.1, 1000 x 1000 at 300 16.4 to 13.1, 4096 x
+  // 4096 at 64 15.1 to 14.0.
+  auto block = [&](int b, auto is_last) {
+    constexpr bool LAST = decltype(is_last)::value;
     const int buf = b & 1;
 #pragma unroll
     for (int k = 0; k < XPT; ++k) *(uint4*)&Xs[buf][xt][xc + 8 * k] = u[k];
-    if (tid < 32) Ss[buf ^ 1][tid] = sal_bytes(sb);
     uint2 cn[RT];
     Planes p[RT];
+    if constexpr (!LAST) {
+      if (tid < 32) Ss[buf ^ 1][tid] = sal_bytes(sb);
 #pragma unroll
-    for (int i = 0; i < RT; ++i) {
-      cn[i] = cw[i];
-      p[i] = planes_of(L[i]);
+      for (int i = 0; i < RT; ++i) {
+        cn[i] = cw[i];
+        p[i] = planes_of(L[i]);
+      }
     }
     __syncthreads();
-    load_x(min(b + 1, b_end - 1));
-    load_codes(min(b + 2, b_end - 1));
-    const uint4 s0 = *(const uint4*)&Ss[buf ^ 1][kq * 8];
-    const uint4 s1 = *(const uint4*)&Ss[buf ^ 1][kq * 8 + 4];
+    uint4 s0, s1;
+    if constexpr (!LAST) {
+      load_x(b + 1);
+      load_codes(min(b + 2, b_end - 1));
+      s0 = *(const uint4*)&Ss[buf ^ 1][kq * 8];
+      s1 = *(const uint4*)&Ss[buf ^ 1][kq * 8 + 4];
+    }
     constexpr int PER = RT * 4 / TG > 0 ? RT * 4 / TG : 1;   // fragments decoded per group
     auto part = [&](int g) {
 #pragma unroll
@@ -767,15 +777,19 @@ __global__ __launch_bounds__(64 * GM_WAVES) void k_gemm_packed(
 #pragma unroll
           for (int i = 0; i < RT; ++i) acc[i][g] = mfma_gv<T8>(a[i][k], xf[g & 1][k], acc[i][g]);
       }
-      part(g);
+      if constexpr (!LAST) part(g);
     }
+    if constexpr (!LAST) {
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
+      for (int i = 0; i < RT; ++i)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) a[i][k] = an[i][k];
+        for (int k = 0; k < 4; ++k) a[i][k] = an[i][k];
+    }
     // the other X buffer is written next; this one is only read again after
-    // the following iteration's barrier
-  }
+    // the following block's barrier
+  };
+  for (int b = b_beg; b + 1 < b_end; ++b) block(b, std::false_type{});
+  if (b_beg < b_end) block(b_end - 1, std::true_type{});
   // acc[i][g][e] = y[token t0 + 16 g + (lane & 15)][row r0 + 16 i + 4 (lane >> 4) + e]
   if constexpr (END) {
     for_ex(end, r0, r0 + 16 * RT, R, C, [&](int r, int c, float d) {
@@ -898,14 +912,17 @@ __global__ __launch_bounds__(256) void k_gemm_packed_sum(const float* __restrict
 // the chip is full; one gives twice the workgroups and a shorter block, which
 // wins where they are few, and is taken if modelled 8 % faster.  Whole linear
 // calls with one / two, each at its own splits (us): 768 x 768 at 17, 64 and
-// 300 tokens 7.7 / 9.1, 9.2 / 10.4, 13.7 / 14.5, 256 x 1024 at 64 11.6 / 17.5,
-// 3072 x 768 at 300 17.8 / 19.2, 4096 x 4096 at 64 and 300 15.4 / 19.5, 41 / 32,
-// 4096 x 16384 at 64 28.8 / 26.9.  Against splits to fill the chip once, twice:
-// 4096 x 16384 at 300 tokens 74 / 83, at 768 167 / 151, 4096 x 4096 at 300 33 /
-// 34, at 768 57 / 65; against no split, 4096 x 1920 at 64 12.1 / 18.3.
+// 300 tokens 7.1 / 8.2, 8.0 / 9.7, 11.4 / 13.7, 256 x 1024 at 64 11.5 / 16.7,
+// 3072 x 768 at 300 14.6 / 18.6, 4096 x 4096 at 64 and 300 14.3 / 18.7, 38.9 /
+// 31.1, 4096 x 16384 at 64 27.6 / 26.4.  Against splits to fill the chip once,
+// twice: 4096 x 16384 at 300 tokens 74 / 83, at 768 167 / 151, 4096 x 4096 at
+// 300 33 / 34, at 768 57 / 65; against no split, 4096 x 1920 at 64 11.1 / 18.4.
+// Over 15 shapes at 17 to 768 tokens the plan is within 10 % of the best of
+// both and 11 splits, but for two at 14 and 24 % (17 and 65 tokens of 6
+// blocks) and the rule below.
 // Products of at most 256 rows, one token tile and 8 blocks take no
 // workspace, as their callers expect (256 x 1024 at 64 tokens 11.6, with
-// splits 8.7).
+// splits 7.1).
 struct GmPlan {
   int tg, rt, tt, ns, bps;
   int64_t row_tiles, tok_tiles;
