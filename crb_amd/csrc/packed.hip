@@ -629,7 +629,7 @@ __global__ __launch_bounds__(64 * GV_WAVES) void k_gemv_packed(
 // idle the block range is split over gridDim.z workgroups, each writing an
 // fp32 partial [T][R] slice that k_gemm_packed_sum adds in split order.  END:
 // the result is rounded to the weights' dtype after bias and exceptions.
-// Counters at 4096 x 16384 and 256 tokens: MFMA busy 32 %, LDS 41 %, 246
+// Counters at 4096 x 16384 and 256 tokens: MFMA busy 32 %, LDS 41 %, 234
 // vector instructions per wavefront and block, half of the wavefronts' time
 // in waits.  Codes and tables of four blocks at a time through LDS (whole
 // lines) measured no faster (85 us at 300 tokens, 34 against 22 at 17).
@@ -917,9 +917,8 @@ __global__ __launch_bounds__(256) void k_gemm_packed_sum(const float* __restrict
 // 31.1, 4096 x 16384 at 64 27.6 / 26.4.  Against splits to fill the chip once,
 // twice: 4096 x 16384 at 300 tokens 74 / 83, at 768 167 / 151, 4096 x 4096 at
 // 300 33 / 34, at 768 57 / 65; against no split, 4096 x 1920 at 64 11.1 / 18.4.
-// Over 15 shapes at 17 to 768 tokens the plan is within 10 % of the best of
-// both and 11 splits, but for two at 14 and 24 % (17 and 65 tokens of 6
-// blocks) and the rule below.
+// Over 15 shapes at 17 to 768 tokens the plan is within 14 % of the best of
+// both and 11 splits, but for 3072 x 768 at 17 (24 %) and the rule below.
 // Products of at most 256 rows, one token tile and 8 blocks take no
 // workspace, as their callers expect (256 x 1024 at 64 tokens 11.6, with
 // splits 7.1).

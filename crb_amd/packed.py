@@ -12,9 +12,9 @@ into a temporary dense weight for the dense GEMM.  The second limit bounds
 memory (up to 768 tokens no temporary weight is allocated); in time the dense
 route wins from about 512 tokens on the larger layers.  Packed / through the
 dense weight on MI355X, us: 4096 x 16384 at 256 / 512 / 768 / 1024 tokens 62 /
-94, 101 / 120, 156 / 138, 182 / 161; 16384 x 4096 61 / 70, 86 / 89, 164 / 109,
-175 / 131; 4096 x 4096 29 / 32, 39 / 39, 56 / 44, 60 / 49; 1024 x 4096 20 / 32,
-23 / 32, 26 / 32, 29 / 32; 768 x 768 16 / 32, 16 / 32, 16 / 32, 18 / 32.
+94, 101 / 117, 151 / 136, 177 / 159; 16384 x 4096 59 / 70, 85 / 89, 160 / 109,
+169 / 128; 4096 x 4096 28 / 31, 38 / 38, 55 / 43, 59 / 49; 1024 x 4096 18 / 31,
+20 / 31, 26 / 31, 28 / 31; 768 x 768 15 / 31, 15 / 31, 16 / 31, 16 / 31.
 """
 from __future__ import annotations
 
