@@ -22,6 +22,10 @@ def _dev_check(*ts):
             raise _lib.CrbqError("crbq tensors must live on the GPU")
 
 
+# torch.cuda.current_stream(device).cuda_stream without the Stream object (1 us)
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _ws(nbytes: int, device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
@@ -526,10 +530,10 @@ def linear_packed(codes: torch.Tensor, lut: torch.Tensor, sal: torch.Tensor, C: 
     lib = _lib.ready(x.device)
     nws = int(lib.crbq_gemm_packed_workspace_size(R, C, T)) if T > 16 else 0
     ws = _ws(nws, x.device) if nws else None
-    ei, _, ed, n = _ex_args(ex, x.device, lut.dtype)
+    ei, _, ed, n = (0, 0, 0, 0) if ex is None else _ex_args(ex, x.device, lut.dtype)
     check(lib.crbq_linear_packed(codes.data_ptr(), codes.stride(0), lut.data_ptr(),
                                  sal.data_ptr(), ei, ed, n, _lib.DTYPES[lut.dtype], R, C,
                                  x.data_ptr(), x.stride(0), T, ptr(bias), y.data_ptr(),
-                                 y.stride(0), ptr(ws), nws, stream_of(y)),
+                                 y.stride(0), ptr(ws), nws, _raw_stream(dev)),
           "crbq_linear_packed")
     return y
