@@ -102,8 +102,8 @@ __device__ __forceinline__ void pack_block(const uint16_t* __restrict__ Q, int64
 #pragma unroll
       for (int s = 0; s < 2; ++s)
         if (grp[s] == G && key[s] > prev) m = min(m, key[s]);
-      m = __builtin_amdgcn_readfirstlane(wave_min_i(m));
-      if (m >= 0x10000) break;
+      m = wave_min_i(m);
+      if (__builtin_amdgcn_readfirstlane(m) >= 0x10000) break;
       cand[k] = m;
       cnt[k] = __popcll(__ballot(grp[0] == G && key[0] == m)) +
                __popcll(__ballot(grp[1] == G && key[1] == m));
@@ -120,10 +120,17 @@ __device__ __forceinline__ void pack_block(const uint16_t* __restrict__ Q, int64
         better += (q < nd && (cnt[q] > cnt[k] || (cnt[q] == cnt[k] && q < k))) ? 1 : 0;
       keep[k] = k < nd && better < cap;
     }
-    int keys[4], found = 0;
+    int keys[4] = {0, 0, 0, 0}, found = 0;
 #pragma unroll
-    for (int k = 0; k < NDV; ++k)
-      if (keep[k] && found < 4) keys[found++] = cand[k];
+    for (int k = 0; k < NDV; ++k) {
+      const bool take = keep[k] && found < 4;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) keys[q] = take && found == q ? cand[k] : keys[q];
+      found += take;
+    }
+    int last = keys[0];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) last = q < found ? keys[q] : last;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       if (grp[s] != G) continue;
@@ -136,7 +143,7 @@ __device__ __forceinline__ void pack_block(const uint16_t* __restrict__ Q, int64
     }
 #pragma unroll
     for (int k = 0; k < cap; ++k)
-      lv[base + k] = found ? unkey16(keys[k < found ? k : found - 1]) : 0u;
+      lv[base + k] = found ? unkey16(k < found ? keys[k] : last) : 0u;
   }
   // exceptions (rare): append to the list
 #pragma unroll
@@ -144,7 +151,10 @@ __device__ __forceinline__ void pack_block(const uint16_t* __restrict__ Q, int64
     if (!exc[s]) continue;
     const int c = b * PB + s * 64 + lane;
     const uint32_t v = unkey16(key[s]);
-    const uint32_t t = lv[(grp[s] == 3 ? 4 : 0) + code[s]];
+    const int at = (grp[s] == 3 ? 4 : 0) + code[s];
+    uint32_t t = lv[0];
+#pragma unroll
+    for (int q = 1; q < 8; ++q) t = at == q ? lv[q] : t;
     const int e = atomicAdd(ex_count, 1);
     if (e < ex_cap) {
       ex_idx[e] = (int64_t)r * C + c;
@@ -192,11 +202,11 @@ __device__ __forceinline__ us2_t row_pk_min(us2_t v) {
 // the minima of key and ~key in the halves of one register) and, for group
 // 3, the smallest and largest of what is left; a block row with an element
 // outside those goes through pack_block, the workgroup's in turn over its
-// wavefronts (768 x 768 with 500 exceptions 104 us; each wavefront its own,
-// 112; 16 wavefronts per workgroup 101, but 295 for 4096 x 16384 without
-// any).  Bound by issue (784 vector instructions per 4 block rows, 84 % of
-// the time busy): with the host's part 88 us for 4096 x 4096, 45 of them the
-// kernel, and 196 for 4096 x 16384, against 357 and 1254 with one wavefront
+// wavefronts (768 x 768 with 500 exceptions 96 us, each wavefront its own
+// 103, on one card; 16 wavefronts a workgroup: 295 for 4096 x 16384 without
+// any).  Bound by issue (753 vector instructions per 4 block rows, 85 % of
+// the time busy): with the host's part 85 us for 4096 x 4096, 43 of them the
+// kernel, and 189 for 4096 x 16384, against 357 and 1254 with one wavefront
 // per block row and eight minimum searches per group.
 constexpr int PK_WAVES = 4;
 __global__ __launch_bounds__(64 * PK_WAVES) void k_pack(const uint16_t* __restrict__ Q, int64_t ldq,
@@ -316,9 +326,10 @@ __global__ __launch_bounds__(64 * PK_WAVES) void k_pack(const uint16_t* __restri
   err = wave_or_i(err);
   if (lane == 0 && err) atomicOr(status, err);
   // block rows with exceptions: the workgroup's, over its wavefronts in turn
+  // (a barrier that does not wait for the stores)
   auto any16 = [&](int k) { return (unsigned)(((sm >> (16 * k)) & 0xffffull) != 0) << k; };
   if (lane == 0) slow4[threadIdx.x >> 6] = any16(0) | any16(1) | any16(2) | any16(3);
-  __syncthreads();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int k = 0;
 #pragma unroll 1
@@ -327,7 +338,9 @@ __global__ __launch_bounds__(64 * PK_WAVES) void k_pack(const uint16_t* __restri
     for (; todo; todo &= todo - 1, ++k) {
       if (k % PK_WAVES != wave) continue;
       const int64_t wi = (int64_t)blockIdx.x * (4 * PK_WAVES) + 4 * q + __builtin_ctz(todo);
-      const int rr = (int)(wi / nblk), bb = (int)(wi - (int64_t)rr * nblk);
+      int rr = (int)(wi / nblk), bb = (int)(wi - (int64_t)rr * nblk);
+      // in vector registers: as scalars their addresses would spill others
+      asm volatile("" : "+v"(rr), "+v"(bb));
       pack_block(Q, ldq, M, ldm, rr, bb, C, nblk, bf16, codes, ldc, lut, ex_idx, ex_val, ex_delta,
                  ex_cap, ex_count, status);
     }
