@@ -209,16 +209,12 @@ __device__ __forceinline__ us2_t row_pk_min(us2_t v) {
 // kernel, and 189 for 4096 x 16384, against 357 and 1254 with one wavefront
 // per block row and eight minimum searches per group.
 constexpr int PK_WAVES = 4;
-__global__ __launch_bounds__(64 * PK_WAVES) void k_pack(const uint16_t* __restrict__ Q, int64_t ldq,
-                                              const uint8_t* __restrict__ M, int64_t ldm,
-                                              int R, int C, int nblk, bool bf16,
-                                              uint8_t* __restrict__ codes, int64_t ldc,
-                                              uint16_t* __restrict__ lut,
-                                              uint8_t* __restrict__ sal,
-                                              int64_t* __restrict__ ex_idx,
-                                              uint16_t* __restrict__ ex_val,
-                                              float* __restrict__ ex_delta, int ex_cap,
-                                              int* ex_count, int* status) {
+__global__ __launch_bounds__(64 * PK_WAVES) void k_pack(
+    const uint16_t* __restrict__ Q, int64_t ldq, const uint8_t* __restrict__ M, int64_t ldm, int R,
+    int C, int nblk, bool bf16, uint8_t* __restrict__ codes, int64_t ldc,
+    uint16_t* __restrict__ lut, uint8_t* __restrict__ sal, int64_t* __restrict__ ex_idx,
+    uint16_t* __restrict__ ex_val, float* __restrict__ ex_delta, int ex_cap, int* ex_count,
+    int* status) {
   __shared__ unsigned slow4[PK_WAVES];
   const int64_t w = (int64_t)blockIdx.x * (4 * PK_WAVES) + (threadIdx.x >> 4);
   const bool live = w < (int64_t)R * nblk;
