@@ -22,10 +22,6 @@ def _dev_check(*ts):
             raise _lib.CrbqError("crbq tensors must live on the GPU")
 
 
-# torch.cuda.current_stream(device).cuda_stream without the Stream object (1 us)
-_raw_stream = torch._C._cuda_getCurrentRawStream
-
-
 def _ws(nbytes: int, device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
@@ -534,6 +530,6 @@ def linear_packed(codes: torch.Tensor, lut: torch.Tensor, sal: torch.Tensor, C: 
     check(lib.crbq_linear_packed(codes.data_ptr(), codes.stride(0), lut.data_ptr(),
                                  sal.data_ptr(), ei, ed, n, _lib.DTYPES[lut.dtype], R, C,
                                  x.data_ptr(), x.stride(0), T, ptr(bias), y.data_ptr(),
-                                 y.stride(0), ptr(ws), nws, _raw_stream(dev)),
+                                 y.stride(0), ptr(ws), nws, stream_of(y)),
           "crbq_linear_packed")
     return y

@@ -826,3 +826,14 @@ def test_block_search_row_split_edges(R):
     candidates spread over many workgroups up to 2048 rows, 16 and 32 rows and
     few workgroups above), against the oracle like the other layouts."""
     test_block_search_candidate_layouts_vs_oracle(R, 50)
+
+
+def test_stream_of_is_torch_current_stream():
+    """The stream handle that every call launches on is torch's current one."""
+    from crb_amd import _lib
+    t = torch.zeros(1, device=DEV)
+    side = torch.cuda.Stream()
+    assert _lib.stream_of(t) == torch.cuda.current_stream(t.device).cuda_stream
+    with torch.cuda.stream(side):
+        assert _lib.stream_of(t) == side.cuda_stream
+    assert _lib.stream_of(t) == torch.cuda.current_stream(t.device).cuda_stream
